@@ -13,15 +13,21 @@ namespace psy {
 //   absent child:   REF_EMPTY
 // Mesh leaves hold 1..3 triangles (src/surface/triangle_mesh.rs:17); instance
 // leaves hold exactly one instance (src/scene/assembly.rs:293).
-// In the device node array bits 28..30 of the first two references (a node
-// always has at least two children) carry the node's 6-bit traversal code,
-// low three bits in child 0, so a static node's visit order comes from the
-// order table without loading the node's last 16 bytes; device code masks
-// them off (child_ref) before following a reference.
+// In the device node array the children sit in slots shaped like the two
+// BVH2 levels the node was collapsed from: slots 0 and 1 under the left child
+// of the top split, 2 and 3 under the right (a side that is one child has it
+// in its first slot).  Any ray's visit order is then three conditional swaps:
+// within each side and of the two sides, each when the ray runs toward
+// negative coordinates along that split's axis.  The axes ride as one-hot
+// bits 28..30: of the top split in slot 0, of the left side's in slot 1, of
+// the right side's in slot 3 (device code drops them before following a
+// reference).  An absent slot is REF_ABSENT and holds a box of +infinity in
+// every plane, which the slab test of a finite ray misses.
 constexpr uint32_t REF_LEAF = 0x80000000u;
 constexpr uint32_t REF_EMPTY = 0xffffffffu;
-constexpr uint32_t REF_CODE_MASK = 0x70000000u;
-constexpr uint32_t REF_CODE_SHIFT = 28;
+constexpr uint32_t REF_AXIS_MASK = 0x70000000u;
+constexpr uint32_t REF_AXIS_SHIFT = 28;
+constexpr uint32_t REF_ABSENT = REF_EMPTY & ~REF_AXIS_MASK;
 constexpr uint32_t MAX_LEAF_FIRST = (1u << 26) - 1;
 constexpr uint32_t MAX_NODES = 1u << 28;
 
@@ -30,9 +36,10 @@ static inline uint32_t make_leaf_ref(uint32_t first, uint32_t count) { return RE
 // One BVH4 node: a 64-B-aligned 128-B record.  The first 96 B are the four
 // child boxes as SoA (BBox4, src/bbox4.rs:16-21) for time sample 0; nodes with
 // time-sampled bounds keep all samples in the motion-bounds array instead.
-//   order[o]  visit order for ray octant o, 2 bits per slot, first child in
-//             the low bits (TRAVERSAL_TABLE[o][traversal_code],
-//             sub_crates/bvh_order, src/accel/bvh4.rs:152-163).
+//   order[o]  visit order of the children for ray octant o, 2 bits per child,
+//             first child in the low bits (TRAVERSAL_TABLE[o][traversal_code],
+//             sub_crates/bvh_order, src/accel/bvh4.rs:152-163), as the
+//             builders leave it; zero in the device form.
 //   meta      bits 0..2 child count, bits 8..15 bounds_len (time samples),
 //             bits 16..21 traversal code.
 //   motion    first BBox4 record of this node's time samples.

@@ -60,18 +60,98 @@ GpuXform to_gpu(const Xf& x) {
     return g;
 }
 
-// Appends `bvh` to the scene arrays, rebasing node and motion indices.
-uint32_t append_bvh(PackedScene& s, const HostBvh4& bvh) {
-    uint32_t node_base = (uint32_t)s.nodes.size();
-    uint32_t motion_base = (uint32_t)s.motion.size();
-    for (GpuNode n : bvh.nodes) {
-        uint32_t cnt = n.meta & 7u;
-        for (uint32_t c = 0; c < cnt; c++)
-            if (!(n.child[c] & REF_LEAF)) n.child[c] += node_base;
-        if (n.motion != REF_EMPTY) n.motion += motion_base;
-        s.nodes.push_back(n);
+// The slots of layout.h for every traversal code: the slots' children (4:
+// absent), the axis bits of their references, and the visit order of the
+// slots per ray octant (TRAVERSAL_TABLE with slots for children, absent
+// slots last).
+struct NodeSlots {
+    uint8_t child[48][4];
+    uint32_t bits[48][4];
+    uint8_t order[8 * 48];
+    NodeSlots() {
+        const uint8_t* table = traversal_order_table();
+        for (uint32_t code = 0; code < 48; code++) {
+            // Axes of the top, left and right splits (3: no split), as the
+            // code packs them (sub_crates/bvh_order/build.rs:5-59).
+            uint32_t top, left = 3, right = 3, cnt = 4;
+            if (code < 27) { top = code % 3; left = (code / 3) % 3; right = code / 9; }
+            else if (code < 36) { cnt = 3; top = (code - 27) % 3; left = (code - 27) / 3; }
+            else if (code < 45) { cnt = 3; top = (code - 36) % 3; right = (code - 36) / 3; }
+            else { cnt = 2; top = code - 45; }
+            const uint32_t at_left = left < 3 ? 2 : 1;  // children under the left side
+            uint32_t slot[4] = {0, 0, 0, 0};
+            for (uint32_t s = 0; s < 4; s++) { child[code][s] = 4; bits[code][s] = 0; }
+            for (uint32_t c = 0; c < cnt; c++) {
+                slot[c] = c < at_left ? c : 2 + c - at_left;
+                child[code][slot[c]] = (uint8_t)c;
+            }
+            auto axis_bits = [](uint32_t axis) { return axis < 3 ? (1u << axis) << REF_AXIS_SHIFT : 0u; };
+            bits[code][0] = axis_bits(top);
+            bits[code][1] = axis_bits(left);
+            bits[code][3] = axis_bits(right);
+            for (uint32_t o = 0; o < 8; o++) {
+                uint32_t v = 0, k = 0;
+                for (; k < cnt; k++) v |= slot[(table[o * 48 + code] >> (2 * k)) & 3u] << (2 * k);
+                for (uint32_t s = 0; s < 4; s++)
+                    if (child[code][s] == 4) v |= s << (2 * k++);
+                order[o * 48 + code] = (uint8_t)v;
+            }
+        }
     }
-    s.motion.insert(s.motion.end(), bvh.motion.begin(), bvh.motion.end());
+};
+const NodeSlots& node_slots() {
+    static const NodeSlots t;
+    return t;
+}
+
+// One sample's four boxes with their children moved to their slots.  Returns
+// whether a plane is NaN.
+bool slot_boxes(const float* in, const uint8_t* child, float* out) {
+    float unordered = 0.0f;  // NaN if a plane is NaN or infinite
+    for (int p = 0; p < 6; p++) {
+        const float v[5] = {in[4 * p], in[4 * p + 1], in[4 * p + 2], in[4 * p + 3], __builtin_huge_valf()};
+        for (int s = 0; s < 4; s++) {
+            out[4 * p + s] = v[child[s]];
+            if (child[s] < 4) unordered += v[child[s]] * 0.0f;
+        }
+    }
+    if (unordered == 0.0f) return false;
+    for (int p = 0; p < 6; p++)
+        for (int s = 0; s < 4; s++)
+            if (out[4 * p + s] != out[4 * p + s]) return true;
+    return false;
+}
+
+// Appends `bvh` to the scene arrays in the device form (layout.h: children
+// in slots), rebasing node and motion indices.
+uint32_t append_bvh(PackedScene& s, const HostBvh4& bvh) {
+    const NodeSlots& t = node_slots();
+    const uint32_t node_base = (uint32_t)s.nodes.size();
+    const uint32_t motion_base = (uint32_t)s.motion.size();
+    s.nodes.resize(s.nodes.size() + bvh.nodes.size());
+    s.motion.resize(s.motion.size() + bvh.motion.size());
+    GpuNode* out = s.nodes.data() + node_base;
+    for (const GpuNode& n : bvh.nodes) {
+        const uint32_t code = (n.meta >> 16) & 0x3fu, blen = (n.meta >> 8) & 0xffu;
+        const uint8_t* child = t.child[code];
+        if (slot_boxes(n.lo_x, child, out->lo_x)) s.nan_boxes = true;
+        for (int k = 0; k < 4; k++) {
+            uint32_t ref = REF_ABSENT;
+            if (child[k] < 4) {
+                ref = n.child[child[k]];
+                if (!(ref & REF_LEAF)) ref += node_base;
+            }
+            out->child[k] = ref | t.bits[code][k];
+        }
+        out->meta = n.meta;
+        out->motion = n.motion;
+        if (n.motion != REF_EMPTY) {
+            out->motion += motion_base;
+            for (uint32_t k = 0; k < blen; k++)
+                if (slot_boxes(bvh.motion[n.motion + k].lo_x, child, s.motion[out->motion + k].lo_x)) s.nan_boxes = true;
+        }
+        out++;
+    }
     if (bvh.root == REF_EMPTY || (bvh.root & REF_LEAF)) return bvh.root;
     return bvh.root + node_base;
 }
@@ -888,19 +968,11 @@ static int pack_flat(const psy_scene_desc* d, Flat& f, PackedScene& s, std::stri
         s.max_stack = need[0] + 2;
     }
 
-    // Device form of the node array: each node's traversal code also rides
-    // in bits 28..30 of its first two child references (layout.h), and the
-    // order table it indexes travels with the scene.
     if (s.nodes.size() > MAX_NODES) {
         err = "the scene's BVHs have more than 2^28 nodes";
         return PSY_E_RANGE;
     }
-    for (GpuNode& n : s.nodes) {
-        const uint32_t code = (n.meta >> 16) & 0x3fu;
-        n.child[0] |= (code & 7u) << REF_CODE_SHIFT;
-        n.child[1] |= (code >> 3) << REF_CODE_SHIFT;
-    }
-    s.order_table.assign(traversal_order_table(), traversal_order_table() + 8 * 48);
+    s.order_table.assign(node_slots().order, node_slots().order + 8 * 48);
     s.build_seconds = std::chrono::duration<double>(std::chrono::steady_clock::now() - t0).count();
     return PSY_OK;
 }

@@ -25,7 +25,7 @@ struct PackedScene {
     std::vector<GpuXform> inv_static;
     std::vector<float> normals;        // xyz per (vertex, time sample), see GpuMesh
     std::vector<uint32_t> nidx;        // stored-order vertex triples per triangle
-    std::vector<uint8_t> order_table;  // TRAVERSAL_TABLE[octant][code], 8 x 48 bytes
+    std::vector<uint8_t> order_table;  // visit order of node slots per [octant][code], 8 x 48 bytes
     uint32_t top_root = REF_EMPTY;
 
     // Lights and shading lookups.
@@ -45,6 +45,7 @@ struct PackedScene {
     bool has_motion = false;    // time-sampled node bounds or vertices
     bool has_lights = false;    // some instance places a light
     bool has_normals = false;   // some mesh has shading normals
+    bool nan_boxes = false;     // some node bound is NaN
     bool nested = false;        // sub-assemblies are traversed as nested BVHs (`groups`)
     uint32_t max_stack = 0;     // deepest pending-node count traversal can need
     uint32_t max_depth = 0;

@@ -28,9 +28,11 @@ struct TraceArgs {
     const GpuRectLight* rect_lights;
     const GpuSphereLight* sphere_lights;
     const float* light_samples;  // time samples of the lights (layout.h)
-    const uint8_t* order_table;  // TRAVERSAL_TABLE[octant][code], 8 x 48 bytes
+    const uint8_t* order_table;  // visit order of node slots per [octant][code], 8 x 48 bytes
     const GpuGroup* groups;      // nested scenes: instance paths (layout.h), else NULL
     uint32_t top_root;
+    uint32_t node_count;
+    uint32_t nan_boxes;          // some node bound is NaN
     // rays (device)
     const float *ox, *oy, *oz, *dx, *dy, *dz, *time, *max_t;
     const uint8_t* flags;

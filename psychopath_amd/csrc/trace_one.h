@@ -109,11 +109,14 @@ __device__ __forceinline__ TraceHit trace_one(const TraceArgs& a, V3 o, V3 d, fl
             const float4* nf = reinterpret_cast<const float4*>(node);
             uint4 refs = *reinterpret_cast<const uint4*>(nf + 6);
             const uint4 tail = *reinterpret_cast<const uint4*>(nf + 7);
-            refs.x &= ~REF_CODE_MASK;  // the traversal code's bits (layout.h)
-            refs.y &= ~REF_CODE_MASK;
+            refs.x &= ~REF_AXIS_MASK;  // the split axes' bits (layout.h)
+            refs.y &= ~REF_AXIS_MASK;
+            refs.w &= ~REF_AXIS_MASK;
             const uint32_t meta = tail.z;
-            const uint32_t cnt = meta & 7u;
             const uint32_t blen = (meta >> 8) & 0xffu;
+            // Visit order of the slots for this ray's octant (loaded before
+            // the box tests, which hide its latency).
+            const uint32_t ord = a.order_table[oct * 48u + ((meta >> 16) & 0x3fu)];
             float4 lx, hx, ly, hy, lz, hz;
             if (blen <= 1) {
                 lx = nf[0]; hx = nf[1]; ly = nf[2]; hy = nf[3]; lz = nf[4]; hz = nf[5];
@@ -136,17 +139,14 @@ __device__ __forceinline__ TraceHit trace_one(const TraceArgs& a, V3 o, V3 d, fl
             }
             uint32_t mask = 0;
             mask |= slab(lx.x, hx.x, ly.x, hy.x, lz.x, hz.x, lo, di, tmax) ? 1u : 0u;
-            mask |= slab(lx.y, hx.y, ly.y, hy.y, lz.y, hz.y, lo, di, tmax) ? 2u : 0u;
+            mask |= slab(lx.y, hx.y, ly.y, hy.y, lz.y, hz.y, lo, di, tmax) && refs.y != REF_ABSENT ? 2u : 0u;
             mask |= slab(lx.z, hx.z, ly.z, hy.z, lz.z, hz.z, lo, di, tmax) ? 4u : 0u;
-            mask |= slab(lx.w, hx.w, ly.w, hy.w, lz.w, hz.w, lo, di, tmax) ? 8u : 0u;
-            mask &= (1u << cnt) - 1u;
+            mask |= slab(lx.w, hx.w, ly.w, hy.w, lz.w, hz.w, lo, di, tmax) && refs.w != REF_ABSENT ? 8u : 0u;
 
-            // Visit order for this ray's octant; push all hit children but the
-            // first in reverse order so the first is visited next.
-            const uint32_t ord = ((oct < 4 ? tail.x : tail.y) >> (8u * (oct & 3u))) & 0xffu;
+            // Push all hit children but the first in reverse order, so the
+            // first is visited next.
             uint32_t next = REF_EMPTY;
             for (int k = 3; k >= 0; --k) {
-                if (k >= (int)cnt) continue;
                 uint32_t c = (ord >> (2 * k)) & 3u;
                 if (mask & (1u << c)) {
                     if (next != REF_EMPTY) T1_PUSH(next);

@@ -36,31 +36,31 @@ constexpr int WAVE = 64;
 // on small scenes.
 constexpr uint32_t CHUNK_MAX = 256;
 
-// Short stack: the newest LDS_DEPTH entries of each lane live in an LDS ring
-// (one column per lane, stride WAVE); when the ring is full the oldest entry
-// moves to a private overflow array and comes back only when the stack
-// unwinds to it, so the pushes and pops of the hot path touch LDS only.
-// `sp` counts entries, entries [0, bot) are in the overflow array.  Macros
-// keep sp and bot in registers (a struct holding the array would live in
-// private memory as a whole).
-#define SSTACK_PUSH(v)                                                    \
-    do {                                                                  \
-        if (sp - bot == LDS_DEPTH) {                                      \
-            spill[bot] = lds_col[(bot % LDS_DEPTH) * WAVE];               \
-            bot++;                                                        \
-        }                                                                 \
-        lds_col[(sp % LDS_DEPTH) * WAVE] = (v);                           \
-        sp++;                                                             \
-    } while (0)
-#define SSTACK_POP(out)                                                   \
-    do {                                                                  \
-        sp--;                                                             \
-        if (sp < bot) {                                                   \
-            bot = sp;                                                     \
-            (out) = spill[sp];                                            \
-        } else {                                                          \
-            (out) = lds_col[(sp % LDS_DEPTH) * WAVE];                     \
-        }                                                                 \
+// Short stack: the newest entries of each lane live in an LDS ring of RING
+// entries (one column per lane, stride WAVE); a node step first moves the
+// oldest entries to a private overflow array until three fit, and they come
+// back only when the stack unwinds to them, so the pushes and pops of the
+// hot path touch LDS only and need no bounds test of their own.  `sp` and
+// `bot` count entries in units of ENTRY, the bytes between two entries of a
+// column; entries [0, bot) are in the overflow array.  Macros keep them in
+// registers (a struct holding the array would live in private memory as a
+// whole).
+constexpr uint32_t ENTRY = WAVE * sizeof(uint32_t);
+#define SSTACK_AT(at) (*reinterpret_cast<uint32_t*>(lds_bytes + (((at) & (RING * ENTRY - ENTRY)) | lane4)))
+#define SSTACK_MAKE_ROOM(k)                             \
+    while (sp - bot > (RING - (k)) * ENTRY) {           \
+        spill[bot / ENTRY] = SSTACK_AT(bot);            \
+        bot += ENTRY;                                   \
+    }
+#define SSTACK_POP(out)                                 \
+    do {                                                \
+        sp -= ENTRY;                                    \
+        if (sp < bot) {                                 \
+            bot = sp;                                   \
+            (out) = spill[sp / ENTRY];                  \
+        } else {                                        \
+            (out) = SSTACK_AT(sp);                      \
+        }                                               \
     } while (0)
 
 // Node parts a static descent step reads: the six box rows and the child
@@ -71,7 +71,7 @@ constexpr uint32_t NODE_PARTS = 7;
 // the assembly applied to the world ray, or the identity at the root
 // (update_local, tracer.rs:65-70, 101-109, 131-148).
 __device__ __forceinline__ void level_local_ray(const TraceArgs& a, const GpuGroup& g, float time, V3 o, V3 d, V3& lo,
-                                                V3& di, uint32_t& oct) {
+                                                V3& di) {
     Xf x = xf_identity();
     if (g.xf_count > 0) {
         uint32_t i1;
@@ -82,32 +82,25 @@ __device__ __forceinline__ void level_local_ray(const TraceArgs& a, const GpuGro
     lo = xf_point(x, o);
     const V3 ld = xf_vector(x, d);
     di = v3(1.0f / ld.x, 1.0f / ld.y, 1.0f / ld.z);
-    oct = octant_of(di);
 }
 
-template <bool COUNT, bool XF, bool MOTION, int LDS_DEPTH, int MIN_WAVES, bool COOP, bool NESTED>
+// RING: LDS stack entries per lane, a power of two.  BIG: the node array is
+// longer than 4 GB, so node addresses take 64-bit offsets.
+template <bool COUNT, bool XF, bool MOTION, uint32_t RING, int MIN_WAVES, bool COOP, bool NESTED, bool BIG>
 __global__ __launch_bounds__(WAVE) __attribute__((amdgpu_waves_per_eu(MIN_WAVES)))
 void trace_persistent_kernel(TraceArgs a, unsigned int* work, uint32_t refill_min, uint32_t leaf_min) {
-    __shared__ uint32_t lds_stack[LDS_DEPTH * WAVE];
+    __shared__ uint32_t lds_stack[RING * WAVE];
     // COOP: the nodes the wave's lanes stand on are fetched by the wave
     // together, consecutive lanes loading consecutive 16-byte parts of one
     // node (one cache line per node instead of one tag lookup per lane and
     // part), staged here and read back by their lanes.
     __shared__ uint4 lds_nodes[COOP ? WAVE * NODE_PARTS : 1];
     __shared__ uint32_t lds_slot[COOP ? WAVE : 1];
-    // TRAVERSAL_TABLE (8 octants x 48 codes): static nodes carry only their
-    // code, in spare bits of their child references (layout.h).
-    __shared__ uint32_t lds_order[8 * 48 / 4];
     const int lane = threadIdx.x;
-    uint32_t* const lds_col = lds_stack + lane;
-    if (!MOTION) {
-        const uint32_t* tab = reinterpret_cast<const uint32_t*>(a.order_table);
-        for (int i = lane; i < 8 * 48 / 4; i += WAVE) lds_order[i] = tab[i];
-        __syncthreads();
-    }
-    const uint8_t* const order_lds = reinterpret_cast<const uint8_t*>(lds_order);
+    const uint32_t lane4 = 4u * (uint32_t)lane;
+    char* const lds_bytes = reinterpret_cast<char*>(lds_stack);
     uint32_t spill[TRACE_STACK_CAPACITY];
-    int sp = 0, bot = 0;
+    uint32_t sp = 0, bot = 0;
 
     const uint32_t n = a.n_dev ? *a.n_dev : (uint32_t)a.n;
     const Xf ident = xf_identity();
@@ -120,10 +113,21 @@ void trace_persistent_kernel(TraceArgs a, unsigned int* work, uint32_t refill_mi
     bool occl = false;
     TriPre pre{};
     V3 lo{}, di{};
-    uint32_t oct = 0;
+    // From the local ray: where on each axis the plane it meets first stands
+    // in a node (0 or 16 bytes on), the split axes it runs down as bits of
+    // REF_AXIS_MASK, and whether slab_finite serves it.
+    uint32_t near_x = 0, near_y = 0, near_z = 0, down = 0;
+    bool finite = false;
+    auto local_ray_set = [&]() {
+        near_x = di.x < 0.0f ? 16u : 0u;
+        near_y = di.y < 0.0f ? 16u : 0u;
+        near_z = di.z < 0.0f ? 16u : 0u;
+        down = octant_of(di) << REF_AXIS_SHIFT;
+        finite = !a.nan_boxes && !(tmax != tmax) && finite_ray(lo, di);
+    };
     uint32_t cur = REF_EMPTY;
     bool in_inst = false;
-    int inst_base = 0;
+    uint32_t inst_base = 0;
     bool has_space = false;
     Xf space;
     uint32_t inst_id = PSY_NONE;
@@ -180,7 +184,7 @@ void trace_persistent_kernel(TraceArgs a, unsigned int* work, uint32_t refill_mi
                     lo = xf_point(ident, o);
                     V3 ld = xf_vector(ident, d);
                     di = v3(1.0f / ld.x, 1.0f / ld.y, 1.0f / ld.z);
-                    oct = octant_of(di);
+                    local_ray_set();
                     pre = tri_precompute(d);
                     cur = a.top_root;
                     sp = 0;
@@ -216,8 +220,6 @@ void trace_persistent_kernel(TraceArgs a, unsigned int* work, uint32_t refill_mi
         // depth-first steps in the same order either way; only their timing
         // changes, so results do not depend on leaf_min.
         //
-        // One descent step of a lane standing on an internal node: its four
-        // child boxes, then the hit children pushed in visit order.
         // The wave's lanes standing on internal nodes (`inner`, ballot `m`)
         // have their nodes' parts loaded by all active lanes together:
         // parts item = slot * 7 + part, item k of a batch by the k-th active
@@ -228,7 +230,7 @@ void trace_persistent_kernel(TraceArgs a, unsigned int* work, uint32_t refill_mi
             const uint32_t items = NODE_PARTS * (uint32_t)__popcll(m);
             const uint64_t act = __ballot(1);
             const uint32_t na = (uint32_t)__popcll(act), ar = (uint32_t)__popcll(act & below);
-            if (inner) lds_slot[slot] = cur;
+            if (inner) lds_slot[slot] = cur & ~REF_AXIS_MASK;
             __syncthreads();
             for (uint32_t base = 0; base < items; base += 4 * na) {
                 uint4 v[4];
@@ -247,95 +249,122 @@ void trace_persistent_kernel(TraceArgs a, unsigned int* work, uint32_t refill_mi
             __syncthreads();
             return slot;
         };
+        // One descent step of a lane standing on an internal node: its four
+        // child boxes, then the hit children pushed in visit order.  The step
+        // is most of the kernel's instructions, and issuing them bounds it
+        // (with the L1's one tag lookup per lane and part): so the planes are
+        // loaded in the order the ray meets them, the box test of finite rays
+        // is min3/max3, and order and pushes take no branches, about 115
+        // vector instructions where a compare-and-select test, a table order
+        // and a branch per child took 230.  16.7M incoherent rays on the
+        // 1M-triangle sphere: 3.98 -> 3.41 ms at 24 waves per CU and leaf_min
+        // 32, 6.77 -> 5.17 ms at 16 and 0.
         auto node_step = [&](uint32_t slot) {
-                const float4* nf = reinterpret_cast<const float4*>(a.nodes + cur);
-                const uint4* staged = lds_nodes + (COOP ? slot * NODE_PARTS : 0u);
-                uint4 refs = COOP ? staged[6] : *reinterpret_cast<const uint4*>(nf + 6);
-                // Static scenes read seven of the node's eight 16-byte parts:
-                // the child count follows from the absent references and the
-                // visit order from the traversal code in the references' spare
-                // bits; time-sampled scenes read the last part for the bounds'
-                // sample count and location.
-                uint4 tail = make_uint4(0u, 0u, 0u, 0u);
-                if (MOTION) tail = *reinterpret_cast<const uint4*>(nf + 7);
-                const uint32_t code = ((refs.x >> REF_CODE_SHIFT) & 7u) | (((refs.y >> REF_CODE_SHIFT) & 7u) << 3);
-                refs.x &= ~REF_CODE_MASK;
-                refs.y &= ~REF_CODE_MASK;
-                const uint32_t cnt =
-                    MOTION ? (tail.z & 7u) : 2u + (refs.z != REF_EMPTY ? 1u : 0u) + (refs.w != REF_EMPTY ? 1u : 0u);
-                float4 lx, hx, ly, hy, lz, hz;
-                const uint32_t blen = MOTION ? ((tail.z >> 8) & 0xffu) : 1u;
-                if (COOP) {
-                    const float4* sf = reinterpret_cast<const float4*>(staged);
-                    lx = sf[0]; hx = sf[1]; ly = sf[2]; hy = sf[3]; lz = sf[4]; hz = sf[5];
-                } else if (!MOTION || blen <= 1) {
-                    lx = nf[0]; hx = nf[1]; ly = nf[2]; hy = nf[3]; lz = nf[4]; hz = nf[5];
-                    if (COUNT) c_nodes++;
-                } else {
-                    uint32_t i1;
-                    float a2;
-                    const float4* m0 = reinterpret_cast<const float4*>(a.motion + tail.w);
-                    if (!lerp_slice_pos(blen, time, i1, a2)) {
-                        m0 += 6 * i1;
-                        lx = m0[0]; hx = m0[1]; ly = m0[2]; hy = m0[3]; lz = m0[4]; hz = m0[5];
-                    } else {
-                        m0 += 6 * i1;
-                        const float4* m1 = m0 + 6;
-                        lx = lerp4(m0[0], m1[0], a2); hx = lerp4(m0[1], m1[1], a2);
-                        ly = lerp4(m0[2], m1[2], a2); hy = lerp4(m0[3], m1[3], a2);
-                        lz = lerp4(m0[4], m1[4], a2); hz = lerp4(m0[5], m1[5], a2);
-                    }
-                    if (COUNT) c_mnodes++;
+            // The node's parts; `toward` gives a plane's distance from the
+            // node's start.
+            const char* const base = reinterpret_cast<const char*>(a.nodes);
+            const uint32_t off = cur << 7;  // drops the axis bits, and the index bits of a BIG scene
+            const char* const big = base + ((uint64_t)(cur & ~REF_AXIS_MASK) << 7);
+            const char* const staged = reinterpret_cast<const char*>(lds_nodes + (COOP ? slot * NODE_PARTS : 0u));
+            auto part = [&](uint32_t plane) {
+                return COOP ? reinterpret_cast<const float4*>(staged + plane)
+                            : reinterpret_cast<const float4*>(BIG ? big + plane : base + (uint64_t)(off + plane));
+            };
+            const uint4 refs = *reinterpret_cast<const uint4*>(part(0) + 6);
+            // Time-sampled scenes also read the last 16 bytes, for the
+            // bounds' sample count and location.
+            uint4 tail = make_uint4(0u, 0u, 0u, 0u);
+            if (MOTION) tail = *reinterpret_cast<const uint4*>(part(0) + 7);
+            const uint32_t blen = MOTION ? ((tail.z >> 8) & 0xffu) : 1u;
+            // The four boxes' planes as the ray meets them: low and high
+            // planes are 16 bytes apart, swapped where the ray runs down.
+            float4 nx, fx, ny, fy, nz, fz;
+            if (!MOTION || blen <= 1) {
+                nx = *part(near_x);               fx = *part(near_x ^ 16u);
+                ny = *(part(near_y) + 2);         fy = *(part(near_y ^ 16u) + 2);
+                nz = *(part(near_z) + 4);         fz = *(part(near_z ^ 16u) + 4);
+                if (COUNT) c_nodes++;
+            } else {
+                uint32_t i1;
+                float a2;
+                const bool between = lerp_slice_pos(blen, time, i1, a2);
+                const float4* m = reinterpret_cast<const float4*>(a.motion + tail.w + i1);
+                float4 lx = m[0], hx = m[1], ly = m[2], hy = m[3], lz = m[4], hz = m[5];
+                if (between) {
+                    m += 6;
+                    lx = lerp4(lx, m[0], a2); hx = lerp4(hx, m[1], a2);
+                    ly = lerp4(ly, m[2], a2); hy = lerp4(hy, m[3], a2);
+                    lz = lerp4(lz, m[4], a2); hz = lerp4(hz, m[5], a2);
                 }
-                uint32_t mask = 0;
-                mask |= slab(lx.x, hx.x, ly.x, hy.x, lz.x, hz.x, lo, di, tmax) ? 1u : 0u;
-                mask |= slab(lx.y, hx.y, ly.y, hy.y, lz.y, hz.y, lo, di, tmax) ? 2u : 0u;
-                mask |= slab(lx.z, hx.z, ly.z, hy.z, lz.z, hz.z, lo, di, tmax) ? 4u : 0u;
-                mask |= slab(lx.w, hx.w, ly.w, hy.w, lz.w, hz.w, lo, di, tmax) ? 8u : 0u;
-                mask &= (1u << cnt) - 1u;
-                const uint32_t ord = MOTION ? ((oct < 4 ? tail.x : tail.y) >> (8u * (oct & 3u))) & 0xffu
-                                            : (uint32_t)order_lds[oct * 48u + code];
-                uint32_t next = REF_EMPTY;
-                for (int k = 3; k >= 0; --k) {
-                    if (k >= (int)cnt) continue;
-                    const uint32_t c = (ord >> (2 * k)) & 3u;
-                    if (mask & (1u << c)) {
-                        if (next != REF_EMPTY) SSTACK_PUSH(next);
-                        next = c == 0 ? refs.x : (c == 1 ? refs.y : (c == 2 ? refs.z : refs.w));
-                    }
-                }
-                cur = next;
-        };
-        if (leaf_min == 0) {
-            // Each lane descends until it stands on a leaf or a dead end.
-            if (COOP) {
-                for (;;) {
-                    const bool inner = cur != REF_EMPTY && !(cur & REF_LEAF);
-                    const uint64_t m = __ballot(inner);
-                    if (m == 0) break;
-                    const uint32_t slot = coop_fetch(inner, m);
-                    if (inner) node_step(slot);
+                nx = near_x ? hx : lx; fx = near_x ? lx : hx;
+                ny = near_y ? hy : ly; fy = near_y ? ly : hy;
+                nz = near_z ? hz : lz; fz = near_z ? lz : hz;
+                if (COUNT) c_mnodes++;
+            }
+            bool h0, h1, h2, h3;
+            if (__ballot(!finite) == 0) {
+                h0 = slab_finite(nx.x, fx.x, ny.x, fy.x, nz.x, fz.x, lo, di, tmax);
+                h1 = slab_finite(nx.y, fx.y, ny.y, fy.y, nz.y, fz.y, lo, di, tmax);
+                h2 = slab_finite(nx.z, fx.z, ny.z, fy.z, nz.z, fz.z, lo, di, tmax);
+                h3 = slab_finite(nx.w, fx.w, ny.w, fy.w, nz.w, fz.w, lo, di, tmax);
+                if (MOTION) {
+                    // lerped planes of an absent slot may be NaN
+                    h1 = h1 && (refs.y | REF_AXIS_MASK) != REF_EMPTY;
+                    h3 = h3 && (refs.w | REF_AXIS_MASK) != REF_EMPTY;
                 }
             } else {
-                while (cur != REF_EMPTY && !(cur & REF_LEAF)) node_step(0u);
+                // Some lane's ray has a zero direction component or the like:
+                // the test in its own operand order, low plane first.
+                // (child by child, so the rare path holds few registers)
+                auto ordered = [&](float na, float fa, float nb, float fb, float nc, float fc) {
+                    const bool h = slab(near_x ? fa : na, near_x ? na : fa, near_y ? fb : nb, near_y ? nb : fb,
+                                        near_z ? fc : nc, near_z ? nc : fc, lo, di, tmax);
+                    __builtin_amdgcn_sched_barrier(0);
+                    return h;
+                };
+                h0 = ordered(nx.x, fx.x, ny.x, fy.x, nz.x, fz.x);
+                h1 = ordered(nx.y, fx.y, ny.y, fy.y, nz.y, fz.y) && (refs.y | REF_AXIS_MASK) != REF_EMPTY;
+                h2 = ordered(nx.z, fx.z, ny.z, fy.z, nz.z, fz.z);
+                h3 = ordered(nx.w, fx.w, ny.w, fy.w, nz.w, fz.w) && (refs.w | REF_AXIS_MASK) != REF_EMPTY;
             }
-        } else {
-            const uint32_t n_active = (uint32_t)__popcll(__ballot(1));
-            for (;;) {
-                if (cur == REF_EMPTY && sp > (in_inst ? inst_base : 0)) SSTACK_POP(cur);
-                const bool inner = cur != REF_EMPTY && !(cur & REF_LEAF);
-                const uint64_t m = __ballot(inner);
-                const uint32_t n_inner = (uint32_t)__popcll(m);
-                if (n_inner == 0 || n_active - n_inner >= leaf_min) break;
-                const uint32_t slot = COOP ? coop_fetch(inner, m) : 0u;
-                if (inner) node_step(slot);
-            }
+            // The hit children in visit order (layout.h): REF_EMPTY where a
+            // slot was missed, then the swaps within and of the two sides.
+            const uint32_t r0 = h0 ? refs.x : REF_EMPTY, r1 = h1 ? refs.y : REF_EMPTY;
+            const uint32_t r2 = h2 ? refs.z : REF_EMPTY, r3 = h3 ? refs.w : REF_EMPTY;
+            const bool swap_l = (refs.y & down) != 0u, swap_r = (refs.w & down) != 0u, swap_t = (refs.x & down) != 0u;
+            const uint32_t l0 = swap_l ? r1 : r0, l1 = swap_l ? r0 : r1;
+            const uint32_t g0 = swap_r ? r3 : r2, g1 = swap_r ? r2 : r3;
+            const uint32_t v0 = swap_t ? g0 : l0, v1 = swap_t ? g1 : l1, v2 = swap_t ? l0 : g0, v3 = swap_t ? l1 : g1;
+            // The first becomes the current node; the others go on the stack,
+            // last first.  Every step stores three entries above the top and
+            // counts those that are real.
+            const bool e0 = v0 != REF_EMPTY, e1 = v1 != REF_EMPTY, e2 = v2 != REF_EMPTY, e3 = v3 != REF_EMPTY;
+            SSTACK_MAKE_ROOM(4);
+            SSTACK_AT(sp) = v3;
+            sp += e3 && (e0 || e1 || e2) ? ENTRY : 0u;
+            SSTACK_AT(sp) = v2;
+            sp += e2 && (e0 || e1) ? ENTRY : 0u;
+            SSTACK_AT(sp) = v1;
+            sp += e1 && e0 ? ENTRY : 0u;
+            cur = e0 ? v0 : e1 ? v1 : e2 ? v2 : v3;
+        };
+        // leaf_min 0: dead ends leave the loop, and it runs until no lane
+        // stands on an internal node.
+        const uint32_t n_active = (uint32_t)__popcll(__ballot(1));
+        for (;;) {
+            if (leaf_min != 0 && cur == REF_EMPTY && sp > (in_inst ? inst_base : 0u)) SSTACK_POP(cur);
+            const bool inner = !(cur & REF_LEAF);
+            const uint64_t m = __ballot(inner);
+            const uint32_t n_inner = (uint32_t)__popcll(m);
+            if (n_inner == 0 || (leaf_min != 0 && n_active - n_inner >= leaf_min)) break;
+            const uint32_t slot = COOP ? coop_fetch(inner, m) : 0u;
+            if (inner) node_step(slot);
         }
 
         // ---- leaf --------------------------------------------------------
         bool finished = false;
         if (cur != REF_EMPTY && (cur & REF_LEAF)) {
-            const uint32_t first = (cur & ~REF_LEAF) >> 2;
+            const uint32_t first = (cur & ~(REF_LEAF | REF_AXIS_MASK)) >> 2;
             const uint32_t count = cur & 3u;
             const uint32_t ii = NESTED ? gbase + first : first;
             if (NESTED && !in_inst && count == 0u) {
@@ -344,18 +373,22 @@ void trace_persistent_kernel(TraceArgs a, unsigned int* work, uint32_t refill_mi
                 grp = first;
                 const GpuGroup g = a.groups[grp];
                 gbase = g.base;
-                level_local_ray(a, g, time, o, d, lo, di, oct);
+                level_local_ray(a, g, time, o, d, lo, di);
+                local_ray_set();
                 cur = REF_EMPTY;
             } else if (NESTED && !in_inst && a.instances[ii].kind == PSY_OBJECT_ASSEMBLY) {
                 // Sub-assembly instance (tracer.rs:95-128): remember the
                 // enclosing path on the stack, move the ray into the
                 // sub-assembly's space and walk its instance BVH.
                 if (COUNT) c_inst++;
-                SSTACK_PUSH(make_level_marker(grp));
+                SSTACK_MAKE_ROOM(1);
+                SSTACK_AT(sp) = make_level_marker(grp);
+                sp += ENTRY;
                 grp = a.instances[ii].mesh;
                 const GpuGroup g = a.groups[grp];
                 gbase = g.base;
-                level_local_ray(a, g, time, o, d, lo, di, oct);
+                level_local_ray(a, g, time, o, d, lo, di);
+                local_ray_set();
                 cur = g.root;
             } else if (!in_inst && XF && a.instances[ii].kind != PSY_OBJECT_MESH) {
                 // Light instance (tracer.rs:95-128 with a light object; light
@@ -374,6 +407,7 @@ void trace_persistent_kernel(TraceArgs a, unsigned int* work, uint32_t refill_mi
                         finished = true;
                     } else {
                         tmax = lt;
+                        finite = finite && lt == lt;
                         kind = PSY_HIT_SURFACE;
                         ht = lt; hb0 = l0; hb1 = l1; hb2 = l2;
                         hprim = lp;
@@ -399,7 +433,7 @@ void trace_persistent_kernel(TraceArgs a, unsigned int* work, uint32_t refill_mi
                         lo = xf_point(x, o);
                         V3 ld = xf_vector(x, d);
                         di = v3(1.0f / ld.x, 1.0f / ld.y, 1.0f / ld.z);
-                        oct = octant_of(di);
+                        local_ray_set();
                         space = inst.xf_count == 1 ? load_xf(a.inv_static + inst.inv_static) : xf_inverse(x);
                         has_space = true;
                     } else {
@@ -461,6 +495,7 @@ void trace_persistent_kernel(TraceArgs a, unsigned int* work, uint32_t refill_mi
                             break;
                         }
                         tmax = t;
+                        finite = finite && t == t;
                         kind = PSY_HIT_SURFACE;
                         ht = t; hb0 = b0; hb1 = b1; hb2 = b2;
                         hprim = prim;
@@ -476,12 +511,13 @@ void trace_persistent_kernel(TraceArgs a, unsigned int* work, uint32_t refill_mi
             if (in_inst && sp == inst_base) {
                 in_inst = false;
                 if (NESTED) {
-                    level_local_ray(a, a.groups[grp], time, o, d, lo, di, oct);
+                    level_local_ray(a, a.groups[grp], time, o, d, lo, di);
+                    local_ray_set();
                 } else if (XF) {
                     lo = xf_point(ident, o);
                     V3 ld = xf_vector(ident, d);
                     di = v3(1.0f / ld.x, 1.0f / ld.y, 1.0f / ld.z);
-                    oct = octant_of(di);
+                    local_ray_set();
                 }
             }
             if (sp == 0) finished = true;
@@ -522,44 +558,49 @@ void trace_persistent_kernel(TraceArgs a, unsigned int* work, uint32_t refill_mi
     }
 }
 
-template <bool COUNT, bool XF, bool MOTION, int D, bool NESTED>
+template <bool COUNT, bool XF, bool MOTION, uint32_t RING, bool NESTED, bool BIG>
 hipError_t launch_one(const TraceArgs& a, unsigned int* work, const TraceTuning& tune, hipStream_t s) {
     // Register budget: 8 waves per SIMD caps the kernel at 64 VGPRs (the
     // compiler keeps the rest in private memory), 4 lets it use up to 128.
     // The cooperative node fetch serves static single-level scenes.
+    auto launch = [&](auto kernel) {
+        hipLaunchKernelGGL(kernel, dim3(tune.waves), dim3(WAVE), 0, s, a, work, tune.refill_min, tune.leaf_min);
+        return hipGetLastError();
+    };
     if constexpr (!COUNT && !MOTION && !NESTED) {
         if (tune.coop) {
-            if (tune.occupancy >= 8)
-                hipLaunchKernelGGL((trace_persistent_kernel<false, XF, false, D, 8, true, false>), dim3(tune.waves),
-                                   dim3(WAVE), 0, s, a, work, tune.refill_min, tune.leaf_min);
-            else
-                hipLaunchKernelGGL((trace_persistent_kernel<false, XF, false, D, 4, true, false>), dim3(tune.waves),
-                                   dim3(WAVE), 0, s, a, work, tune.refill_min, tune.leaf_min);
-            return hipGetLastError();
+            if (tune.occupancy >= 8) return launch(trace_persistent_kernel<false, XF, false, RING, 8, true, false, false>);
+            return launch(trace_persistent_kernel<false, XF, false, RING, 4, true, false, false>);
         }
     }
-    if (!COUNT && tune.occupancy >= 8)
-        hipLaunchKernelGGL((trace_persistent_kernel<COUNT, XF, MOTION, D, 8, false, NESTED>), dim3(tune.waves), dim3(WAVE), 0,
-                           s, a, work, tune.refill_min, tune.leaf_min);
-    else
-        hipLaunchKernelGGL((trace_persistent_kernel<COUNT, XF, MOTION, D, 4, false, NESTED>), dim3(tune.waves), dim3(WAVE), 0,
-                           s, a, work, tune.refill_min, tune.leaf_min);
-    return hipGetLastError();
+    if constexpr (!COUNT && !BIG) {
+        if (tune.occupancy >= 8) return launch(trace_persistent_kernel<false, XF, MOTION, RING, 8, false, NESTED, false>);
+    }
+    return launch(trace_persistent_kernel<COUNT, XF, MOTION, RING, 4, false, NESTED, BIG>);
 }
 
 template <bool COUNT, bool XF, bool MOTION, bool NESTED>
 hipError_t launch_depth(const TraceArgs& a, unsigned int* work, const TraceTuning& tune, hipStream_t s) {
-    if (COUNT || NESTED) return launch_one<COUNT, XF, MOTION, 16, NESTED>(a, work, tune, s);
-    switch (tune.lds_depth) {
-        case 8: return launch_one<COUNT, XF, MOTION, 8, false>(a, work, tune, s);
-        case 24: return launch_one<COUNT, XF, MOTION, 24, false>(a, work, tune, s);
-        default: return launch_one<COUNT, XF, MOTION, 16, false>(a, work, tune, s);
+    if constexpr (COUNT || NESTED) {
+        return launch_one<COUNT, XF, MOTION, 16, NESTED, false>(a, work, tune, s);
+    } else {
+        switch (tune.lds_depth) {
+            case 8: return launch_one<COUNT, XF, MOTION, 8, false, false>(a, work, tune, s);
+            case 24: return launch_one<COUNT, XF, MOTION, 32, false, false>(a, work, tune, s);
+            default: return launch_one<COUNT, XF, MOTION, 16, false, false>(a, work, tune, s);
+        }
     }
 }
 
 template <bool COUNT>
 hipError_t launch_feat(const TraceArgs& a, unsigned int* work, const TraceTuning& tune, bool xf, bool motion,
                        hipStream_t s) {
+    // More than 4 GB of nodes: the most general build, with 64-bit node
+    // offsets.
+    if (a.node_count > (1u << 25)) {
+        if (a.groups) return launch_one<COUNT, true, true, 16, true, true>(a, work, tune, s);
+        return launch_one<COUNT, true, true, 16, false, true>(a, work, tune, s);
+    }
     // Nested scenes take the transform path, with or without time samples.
     if (a.groups) {
         if (motion) return launch_depth<COUNT, true, true, true>(a, work, tune, s);
