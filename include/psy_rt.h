@@ -249,8 +249,8 @@ typedef struct {
  * reading consecutive parts of one node, staged in LDS and read back, for
  * scenes without time samples (elsewhere it runs as the persistent kernel).
  * The persistent kernel keeps
- * `waves_per_cu` wave64 workgroups per compute unit resident, each taking
- * chunks of rays from a global counter; lanes whose ray finished are
+ * `waves_per_cu` wave64 workgroups per compute unit resident, each starting
+ * on its share of the rays and then taking chunks from a counter; lanes whose ray finished are
  * refilled from the wave's chunk once `refill_min` lanes of a wave are idle; `stack_lds` stack entries per lane
  * live in LDS (8, 16 or 24) and the rest in private memory; `simd_waves`
  * is the register budget, as resident waves per SIMD (4: up to 128 VGPRs,
@@ -360,12 +360,12 @@ int psy_finalize_hits(psy_tracer* tracer, const psy_ray_soa* rays, uint64_t n, c
  * `stream` (a hipStream_t, NULL for the default stream) and not waited for.
  * The scene must already be resident on the current device (creating a
  * tracer for it uploads it).  `tuning` may be NULL (the tracer's default
- * shape); the simple kernel is not offered.  The one scratch word the
- * persistent kernels need (their ray counter) lives in a fixed
+ * shape); the simple kernel is not offered.  The scratch the persistent
+ * kernels need (their ray counters) lives in a fixed
  * PSY_NOALLOC_SCRATCH_BYTES device array of the library, one per device and
  * shared by every call on it: calls that overlap on one device race.  At
  * most PSY_NOALLOC_MAX_RAYS rays per call (PSY_E_RANGE beyond). */
-#define PSY_NOALLOC_SCRATCH_BYTES 256u
+#define PSY_NOALLOC_SCRATCH_BYTES 1024u
 #define PSY_NOALLOC_MAX_RAYS 0x7fffffffull
 int psy_trace_noalloc(const psy_scene* scene, const psy_ray_soa* rays, uint64_t n, psy_hit_soa* hits,
                       const psy_trace_tuning* tuning, void* stream);

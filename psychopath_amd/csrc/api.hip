@@ -315,7 +315,7 @@ int psy_tracer_create(const psy_scene* scene, uint64_t max_batch, psy_tracer** o
     if (e == hipSuccess) e = hipEventCreate(&t->ev0);
     if (e == hipSuccess) e = hipEventCreate(&t->ev1);
     if (e == hipSuccess) e = hipMalloc((void**)&t->counters, 8 * sizeof(unsigned long long));
-    if (e == hipSuccess) e = hipMalloc((void**)&t->work, 64);
+    if (e == hipSuccess) e = hipMalloc((void**)&t->work, TRACE_WORK_WORDS * sizeof(unsigned int));
     if (e != hipSuccess) {
         delete t;
         return fail(PSY_E_DEVICE, std::string("tracer setup: ") + hipGetErrorString(e));

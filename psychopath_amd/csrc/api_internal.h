@@ -80,7 +80,7 @@ struct psy_tracer {
     // device staging for host-memory calls: 8 ray floats + flags, hit fields
     void* staging = nullptr;
     unsigned long long* counters = nullptr;
-    unsigned int* work = nullptr;   // persistent-kernel ray counter
+    unsigned int* work = nullptr;   // the persistent kernels' ray counters
     psy_trace_tuning tuning{PSY_KERNEL_PERSISTENT, 16, 16, 16, 4};
     uint32_t cu_count = 256;
 

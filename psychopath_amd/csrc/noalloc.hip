@@ -3,13 +3,13 @@
 // memory (code under HIP graph capture, tight serving loops, hosts that
 // forbid hipMalloc after set-up).
 //
-// The persistent traversal kernel needs one scratch word: the ray counter its
-// waves take rays from.  psy_trace keeps it in the tracer's allocation; here
-// it lives in `scratch`, a fixed device array of this library.  Each device
+// The persistent traversal kernels need a little scratch: the ray counters
+// their waves take rays from.  psy_trace keeps them in the tracer's allocation;
+// here they live in `scratch`, a fixed device array of this library.  Each device
 // holds its own copy of the array at its own address, looked up once per
 // device with hipGetSymbolAddress; host code only ever passes that address.
 // Calls on one device share the array, so calls that overlap on one device
-// (two streams, or two host threads) race on the counter.
+// (two streams, or two host threads) race on the counters.
 #include <hip/hip_runtime.h>
 
 #include <mutex>
@@ -22,8 +22,9 @@ using namespace psy::api;
 
 namespace {
 
-// Scratch of psy_trace_noalloc, per device.  Word 0: the persistent
-// kernel's ray counter, reset by a kernel at the start of every call.
+// Scratch of psy_trace_noalloc, per device: the persistent kernels' ray
+// counters, reset by a kernel at the start of every call.
+static_assert(PSY_NOALLOC_SCRATCH_BYTES >= TRACE_WORK_WORDS * sizeof(unsigned int), "scratch holds the ray counters");
 static __device__ __align__(256) unsigned int scratch[PSY_NOALLOC_SCRATCH_BYTES / sizeof(unsigned int)];
 
 constexpr int MAX_DEVICES = 64;

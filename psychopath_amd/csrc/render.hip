@@ -1141,7 +1141,7 @@ int enqueue_wave(psy_renderer* r, uint32_t steps) {
             rc = trace(qa_in, r->ha, false, r->work, ST_TRACE);
             if (rc) return rc;
         }
-        rc = trace(qs_in, r->hs, true, r->work + 16, ST_SHADOW_TRACE);
+        rc = trace(qs_in, r->hs, true, r->work + TRACE_WORK_WORDS, ST_SHADOW_TRACE);
         if (!rc) rc = staged(r, ST_SHADOW, [&]() -> int {
             hipLaunchKernelGGL(shadow_kernel, dim3(grid), dim3(KBLOCK), 0, s, qs_in, r->hs.kind, r->P, r->sc.rays);
             PSY_HIP(hipGetLastError());
@@ -1450,7 +1450,7 @@ int psy_renderer_create(const psy_scene* scene_c, const psy_world_desc* world, u
     if (!rc) rc = r->alloc(&r->order, C);
     if (!rc) rc = r->alloc(&r->counts, COUNTS_WORDS);
     if (!rc) rc = r->alloc(&r->wave_idx, 1);
-    if (!rc) rc = r->alloc(&r->work, 64);
+    if (!rc) rc = r->alloc(&r->work, 2 * TRACE_WORK_WORDS);
     if (!rc) rc = r->alloc(&r->prof_dev, 16);
     if (!rc && hipMemset(r->prof_dev, 0, 16 * sizeof(unsigned long long)) != hipSuccess)
         rc = fail(PSY_E_DEVICE, "profile counters");

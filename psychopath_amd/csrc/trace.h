@@ -16,6 +16,12 @@ constexpr int TRACE_LDS_DEPTH = 24;        // stack entries per lane held in LDS
 // a binary depth of at most 42: src/accel/bvh_base.rs:7, bvh4.rs:87).
 constexpr int TRACE_STACK_CAPACITY = 3 * (22 + 22) + 2;
 
+// The persistent kernels take their rays from TRACE_RANGES counters, one per
+// XCD's worth of waves and TRACE_RANGE_WORDS words apart (a cache line each).
+constexpr uint32_t TRACE_RANGES = 8;
+constexpr uint32_t TRACE_RANGE_WORDS = 32;
+constexpr uint32_t TRACE_WORK_WORDS = TRACE_RANGES * TRACE_RANGE_WORDS;
+
 struct TraceArgs {
     // scene
     const GpuNode* nodes;
@@ -62,8 +68,8 @@ struct TraceTuning {
 // One lane per ray, one launch-wide grid (trace.hip).
 hipError_t launch_trace(const TraceArgs& args, bool counted, hipStream_t stream);
 
-// Persistent waves with lane refill (trace_persistent.hip).  `work` is a
-// device counter the launch resets.
+// Persistent waves with lane refill (trace_persistent.hip).  `work`:
+// TRACE_WORK_WORDS device words, the ray counters, which the launch resets.
 hipError_t launch_trace_persistent(const TraceArgs& args, bool counted, bool has_xf, bool has_motion,
                                    unsigned int* work, const TraceTuning& tune, hipStream_t stream);
 

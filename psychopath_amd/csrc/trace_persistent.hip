@@ -4,10 +4,11 @@
 // order, src/accel/bvh4.rs:101-184, with the same box and triangle tests),
 // reorganised for throughput on incoherent rays:
 //   * one wave64 per workgroup, launched only as many waves as the chip holds
-//     at once; each wave keeps taking chunks of rays from a global counter;
+//     at once; each wave starts on its share of the rays and then keeps
+//     taking chunks from a counter (one per range of rays);
 //   * lanes whose ray finished are refilled in bulk once at least
 //     `refill_min` lanes of the wave are idle, from the wave's chunk (an
-//     atomic only when the chunk runs short), the new rays spread over the
+//     atomic only when the chunk is used up), the new rays spread over the
 //     idle lanes by a ballot prefix count;
 //   * the traversal is "while-while": lanes descend internal nodes (popping
 //     past dead ends) until the whole wave stands on leaves, then run the
@@ -29,12 +30,44 @@ namespace psy {
 namespace {
 
 constexpr int WAVE = 64;
-// Most rays a wave takes from the global counter at once.  Larger chunks
+// Most rays a wave takes from a counter at once.  Larger chunks
 // spread the rays in flight over a wider stretch of the queue: on queues in
 // pixel order (a renderer's camera and bounce rays) that costs coherence, 4%
-// on the large instanced scene at 512, while 64 leaves the counter contended
+// on the large instanced scene at 512, while 64 leaves the counters contended
 // on small scenes.
 constexpr uint32_t CHUNK_MAX = 256;
+
+// The rays are dealt to TRACE_RANGES ranges in blocks of RANGE_BLOCK rays,
+// round robin, and wave w starts on range w % TRACE_RANGES, on a share that
+// needs no counter.  One counter for all rays cost its waves their turn on
+// one address, about 12 ns each: 49 us for a launch without rays, while a
+// launch with few ran them 64 to a wave on a corner of the chip.  4,096 rays
+// on the 65,536-triangle sphere: 174 -> 122 us; the Cornell box at 64x64, 4
+// spp: 1.27 -> 0.75 ms; the large scene at full HD, whose later bounces are
+// small launches: 15.1 -> 12.5 ms.  Blocks of 512 rays time the same or 1-2%
+// more and of 4,096 up to 9% more (coherent rays: less balance, no more
+// locality).  Ray k of range x:
+constexpr uint32_t RANGE_BITS = 6;
+constexpr uint32_t RANGE_BLOCK = 1u << RANGE_BITS;
+__device__ __forceinline__ uint32_t range_ray(uint32_t x, uint32_t k) {
+    return (((k >> RANGE_BITS) * TRACE_RANGES + x) << RANGE_BITS) + (k & (RANGE_BLOCK - 1u));
+}
+// Rays of range x; range 0 is never the shorter.
+__host__ __device__ __forceinline__ uint32_t range_count(uint32_t n, uint32_t x) {
+    const uint32_t round = RANGE_BLOCK * TRACE_RANGES, rest = n % round, before = x * RANGE_BLOCK;
+    const uint32_t part = rest < before ? 0u : rest - before;
+    return (n / round) * RANGE_BLOCK + (part < RANGE_BLOCK ? part : RANGE_BLOCK);
+}
+// Rays of its range each wave starts on without asking a counter: all of
+// them where that is at most one ray per lane, spread evenly over the waves;
+// else half of an even share, and the rest comes from the counters.
+__host__ __device__ __forceinline__ uint32_t first_rays(uint32_t n, uint32_t waves) {
+    const uint32_t per_range = waves / TRACE_RANGES;
+    const uint32_t share = (range_count(n, 0) + per_range - 1u) / per_range;
+    if (share <= (uint32_t)WAVE) return share;
+    const uint32_t half = share / 2u;
+    return half < (uint32_t)WAVE ? (uint32_t)WAVE : half < CHUNK_MAX ? half : CHUNK_MAX;
+}
 
 // Short stack: the newest entries of each lane live in an LDS ring of RING
 // entries (one column per lane, stride WAVE); a node step first moves the
@@ -138,42 +171,64 @@ void trace_persistent_kernel(TraceArgs a, unsigned int* work, uint32_t refill_mi
     float ht = 0.0f, hb0 = 0.0f, hb1 = 0.0f, hb2 = 0.0f;
     uint32_t hprim = PSY_NONE, hinst = PSY_NONE;
     uint64_t c_nodes = 0, c_mnodes = 0, c_tris = 0, c_mtris = 0, c_inst = 0;
-    bool exhausted = false;
-    // The wave's chunk: rays [next, end) taken from the counter and not yet
-    // handed to a lane; `seen` is where the counter stood after the wave's
-    // last fetch, and `drained` that it had passed n then.
-    uint32_t next = 0, end = 0, seen = 0;
-    bool drained = false;
+    // The wave's chunk: rays [next, end) of range rx taken and not yet handed
+    // to a lane.  Rays below `dealt` of every range are the waves' first
+    // chunks; the counter of a range counts on from there.  `seen`: where
+    // rx's counter stood when last looked at; `drained`: every range's rays
+    // are taken.
+    const uint32_t per_range = gridDim.x / TRACE_RANGES;
+    const uint32_t first = first_rays(n, gridDim.x);
+    const uint32_t dealt = first * per_range;
+    uint32_t rx = blockIdx.x % TRACE_RANGES, seen = 0;
+    uint32_t next = min((blockIdx.x / TRACE_RANGES) * first, range_count(n, rx));
+    uint32_t end = min(next + first, range_count(n, rx));
+    bool drained = dealt >= range_count(n, 0);
+    bool exhausted = drained && next == end;
 
     for (;;) {
         // ---- refill idle lanes ------------------------------------------
-        // Idle lanes take the rest of the wave's chunk first; one atomic
-        // fetches a new chunk only when the rest is short, sized by guided
-        // self-scheduling (the remaining rays over 2x the waves, at most
-        // CHUNK_MAX), so the counter sees few atomics while the last rays
-        // still spread over all waves.
+        // Idle lanes take the rest of the wave's chunk first; when it is
+        // used up one atomic fetches another, sized by guided
+        // self-scheduling (the range's remaining rays over 2x its waves, at
+        // most CHUNK_MAX), so the counters see few atomics while the last
+        // rays still spread over all waves.  A wave whose range is used up
+        // goes on with the next one that is not.
         const uint64_t idle = __ballot(!has);
         if (!exhausted && (uint32_t)__popcll(idle) >= refill_min) {
             const uint32_t want = (uint32_t)__popcll(idle);
-            const uint32_t avail = end - next;
-            uint32_t fresh = 0, fresh_end = 0;
-            if (avail < want && !drained) {
-                const int leader = __ffsll((unsigned long long)idle) - 1;
-                const uint32_t left = n > seen ? n - seen : 0u;
-                const uint32_t take =
-                    max(want - avail, min(left / (2u * (uint32_t)gridDim.x), (uint32_t)CHUNK_MAX));
-                if (lane == leader) fresh = atomicAdd(work, take);
-                fresh = __shfl(fresh, leader);
-                seen = fresh + take;
-                drained = seen >= n;
-                fresh_end = fresh < n ? min(seen, n) : fresh;
+            while (next == end && !drained) {
+                const uint32_t count = range_count(n, rx);
+                const uint32_t left = count > dealt + seen ? count - dealt - seen : 0u;
+                if (left != 0u) {
+                    const uint32_t take = max(want, min(left / (2u * per_range), (uint32_t)CHUNK_MAX));
+                    uint32_t at = 0;
+                    if (lane == 0) at = atomicAdd(work + rx * TRACE_RANGE_WORDS, take);
+                    at = __builtin_amdgcn_readfirstlane(at);
+                    seen = at + take;
+                    next = min(dealt + at, count);
+                    end = min(dealt + at + take, count);
+                } else {
+                    uint32_t at = 0;
+                    bool open = false;
+                    if (lane < (int)TRACE_RANGES) {
+                        at = __hip_atomic_load(work + lane * TRACE_RANGE_WORDS, __ATOMIC_RELAXED,
+                                               __HIP_MEMORY_SCOPE_AGENT);
+                        open = dealt + at < range_count(n, (uint32_t)lane);
+                    }
+                    const uint32_t m = (uint32_t)__ballot(open);
+                    drained = m == 0u;
+                    // the first open range after rx, round robin
+                    const uint32_t turned = (m | (m << TRACE_RANGES)) >> (rx + 1u);
+                    if (!drained) rx = (rx + (uint32_t)__ffs(turned)) % TRACE_RANGES;
+                    seen = (uint32_t)__shfl((int)at, (int)rx);
+                }
             }
+            const uint32_t avail = end - next;
             if (!has) {
                 const uint32_t rank = (uint32_t)__popcll(idle & ((1ull << lane) - 1ull));
-                const uint32_t mine = rank < avail ? next + rank : fresh + (rank - avail);
-                if (rank < avail || mine < fresh_end) {
+                if (rank < avail) {
                     has = true;
-                    ray = mine;
+                    ray = range_ray(rx, next + rank);
                     o = v3(a.ox[ray], a.oy[ray], a.oz[ray]);
                     d = v3(a.dx[ray], a.dy[ray], a.dz[ray]);
                     time = MOTION || XF ? a.time[ray] : 0.0f;
@@ -195,17 +250,13 @@ void trace_persistent_kernel(TraceArgs a, unsigned int* work, uint32_t refill_mi
                     kind = PSY_HIT_MISS;
                 }
             }
-            if (avail >= want) {
-                next += want;
-            } else {
-                // The lanes took the whole rest and the head of the new chunk
-                // (none when the counter had already passed n).
-                next = min(fresh + (want - avail), fresh_end);
-                end = fresh_end;
-            }
+            next += min(want, avail);
             exhausted = drained && next == end;
         }
-        if (__ballot(has) == 0) break;
+        if (__ballot(has) == 0) {
+            if (exhausted) break;
+            continue;
+        }
         if (!has) continue;
 
         // ---- descend internal nodes ---------------------------------------
@@ -614,19 +665,25 @@ hipError_t launch_feat(const TraceArgs& a, unsigned int* work, const TraceTuning
 
 }  // namespace
 
-// Sets *work = 0 with a kernel, so the launch sequence can be captured in a
-// graph (no memset node).
-__global__ void reset_work_kernel(unsigned int* work) { *work = 0u; }
+// Zeroes the ranges' counters with a kernel, so the launch sequence can be
+// captured in a graph (no memset node).
+__global__ void reset_work_kernel(unsigned int* work) { work[threadIdx.x * TRACE_RANGE_WORDS] = 0u; }
 
 hipError_t launch_trace_persistent(const TraceArgs& args, bool counted, bool has_xf, bool has_motion,
-                                   unsigned int* work, const TraceTuning& tune, hipStream_t stream) {
+                                   unsigned int* work, const TraceTuning& tuning, hipStream_t stream) {
     if (args.n == 0) return hipSuccess;
+    TraceTuning tune = tuning;
+    tune.waves = (tune.waves + TRACE_RANGES - 1u) / TRACE_RANGES * TRACE_RANGES;
     if (args.n >= 0x80000000ull || tune.waves == 0 || tune.refill_min == 0 || tune.refill_min > 64 ||
         tune.leaf_min > 64)
         return hipErrorInvalidValue;
-    hipLaunchKernelGGL(reset_work_kernel, dim3(1), dim3(1), 0, stream, work);
-    hipError_t e = hipGetLastError();
-    if (e != hipSuccess) return e;
+    // A launch whose waves start on all of its rays reads no counter.
+    const uint32_t n = (uint32_t)args.n;
+    if (args.n_dev || (uint64_t)first_rays(n, tune.waves) * (tune.waves / TRACE_RANGES) < range_count(n, 0)) {
+        hipLaunchKernelGGL(reset_work_kernel, dim3(1), dim3(TRACE_RANGES), 0, stream, work);
+        hipError_t e = hipGetLastError();
+        if (e != hipSuccess) return e;
+    }
     return counted ? launch_feat<true>(args, work, tune, has_xf, has_motion, stream)
                    : launch_feat<false>(args, work, tune, has_xf, has_motion, stream);
 }
