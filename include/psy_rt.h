@@ -249,7 +249,8 @@ typedef struct {
  * reading consecutive parts of one node, staged in LDS and read back, for
  * scenes without time samples (elsewhere it runs as the persistent kernel).
  * The persistent kernel keeps
- * `waves_per_cu` wave64 workgroups per compute unit resident, each starting
+ * `waves_per_cu` wave64 workgroups per compute unit resident (at most as
+ * many as its registers and LDS let a unit hold), each starting
  * on its share of the rays and then taking chunks from a counter; lanes whose ray finished are
  * refilled from the wave's chunk once `refill_min` lanes of a wave are idle; `stack_lds` stack entries per lane
  * live in LDS (8, 16 or 24) and the rest in private memory; `simd_waves`

@@ -84,7 +84,7 @@ int device_cu_count(uint32_t& cus_out) {
 hipError_t launch_tuned(const psy_scene* scene, const psy_trace_tuning& tuning, uint32_t cu_count, unsigned int* work,
                         const TraceArgs& a, bool counted, hipStream_t stream) {
     if (tuning.kernel == PSY_KERNEL_SIMPLE) return launch_trace(a, counted, stream);
-    TraceTuning tt{cu_count * tuning.waves_per_cu, tuning.refill_min, tuning.stack_lds, tuning.simd_waves,
+    TraceTuning tt{cu_count, tuning.waves_per_cu, tuning.refill_min, tuning.stack_lds, tuning.simd_waves,
                    tuning.leaf_min, tuning.kernel == PSY_KERNEL_PERSISTENT_COOP ? 1u : 0u};
     return launch_trace_persistent(a, counted, scene->host.has_xf || scene->host.has_lights, scene->host.has_motion,
                                    work, tt, stream);

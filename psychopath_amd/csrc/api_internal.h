@@ -24,6 +24,17 @@ int fail(int code, const std::string& msg);
             return ::psy::api::fail(PSY_E_DEVICE, std::string(#call) + ": " + hipGetErrorString(e_));         \
     } while (0)
 
+// The launch shape of a new tracer or renderer: as many waves as the kernel's
+// build allows on a CU (24 is more than any 4-wave build does, 20 on static
+// scenes and 16 with transforms), and descent rounds that end when half of a
+// wave waits.  Against 16 waves and descents to the last lane: 16.7M
+// incoherent rays on the 1M-triangle sphere 5.15 -> 3.37 ms, 4.0M shadow rays
+// 1.28 -> 0.93 ms, 1M rays on the motion scene 1.63 -> 1.36 ms and its
+// 960x540 render 18.2 -> 16.4 ms, the large scene at full HD 12.5 -> 12.1 ms,
+// the Cornell box 7.87 -> 7.87 ms.  leaf_min 24 is 2% faster on the motion
+// scene and 3% slower on the sphere; 40 the other way round.
+inline psy_trace_tuning default_tuning() { return psy_trace_tuning{PSY_KERNEL_PERSISTENT, 24, 16, 16, 4, 32}; }
+
 template <typename T>
 int upload(const std::vector<T>& v, T** out) {
     *out = nullptr;
@@ -81,7 +92,7 @@ struct psy_tracer {
     void* staging = nullptr;
     unsigned long long* counters = nullptr;
     unsigned int* work = nullptr;   // the persistent kernels' ray counters
-    psy_trace_tuning tuning{PSY_KERNEL_PERSISTENT, 16, 16, 16, 4};
+    psy_trace_tuning tuning = psy::api::default_tuning();
     uint32_t cu_count = 256;
 
     ~psy_tracer() {

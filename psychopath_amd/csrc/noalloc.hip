@@ -65,7 +65,7 @@ extern "C" int psy_trace_noalloc(const psy_scene* scene, const psy_ray_soa* rays
     if (!scene) return fail(PSY_E_INVALID, "scene is NULL");
     int rc = check_soa(rays, hits);
     if (rc) return rc;
-    psy_trace_tuning t{PSY_KERNEL_PERSISTENT, 16, 16, 16, 4, 0};
+    psy_trace_tuning t = default_tuning();
     if (tuning) {
         rc = check_tuning(tuning);
         if (rc) return rc;

@@ -161,7 +161,7 @@ struct psy_renderer {
     hipEvent_t ev0 = nullptr, ev1 = nullptr;
     uint64_t capacity = 0;
     uint32_t cu_count = 256;
-    psy_trace_tuning tuning{PSY_KERNEL_PERSISTENT, 16, 16, 16, 4};
+    psy_trace_tuning tuning = psy::api::default_tuning();
     bool use_graphs = true;
     bool sort_materials = true;
     bool plain = false;  // one megakernel launch per render

@@ -107,19 +107,23 @@ const NodeSlots& node_slots() {
 // One sample's four boxes with their children moved to their slots.  Returns
 // whether a plane is NaN.
 bool slot_boxes(const float* in, const uint8_t* child, float* out) {
-    float unordered = 0.0f;  // NaN if a plane is NaN or infinite
-    for (int p = 0; p < 6; p++) {
-        const float v[5] = {in[4 * p], in[4 * p + 1], in[4 * p + 2], in[4 * p + 3], __builtin_huge_valf()};
-        for (int s = 0; s < 4; s++) {
-            out[4 * p + s] = v[child[s]];
-            if (child[s] < 4) unordered += v[child[s]] * 0.0f;
-        }
+    const float inf = __builtin_huge_valf();
+    bool nan = false;
+    for (int k = 0; k < 24; k++) nan |= in[k] != in[k];
+    if (child[1] == 1) {  // the left side has two children: slots as children
+        std::memcpy(out, in, 24 * sizeof(float));
+        if (child[3] == 4)
+            for (int p = 0; p < 6; p++) out[4 * p + 3] = inf;
+        return nan;
     }
-    if (unordered == 0.0f) return false;
-    for (int p = 0; p < 6; p++)
-        for (int s = 0; s < 4; s++)
-            if (out[4 * p + s] != out[4 * p + s]) return true;
-    return false;
+    const bool two = child[3] == 4;
+    for (int p = 0; p < 6; p++) {
+        out[4 * p] = in[4 * p];
+        out[4 * p + 1] = inf;
+        out[4 * p + 2] = in[4 * p + 1];
+        out[4 * p + 3] = two ? inf : in[4 * p + 2];
+    }
+    return nan;
 }
 
 // Appends `bvh` to the scene arrays in the device form (layout.h: children

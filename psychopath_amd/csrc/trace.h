@@ -57,7 +57,8 @@ struct TraceArgs {
 
 // Launch shape of the persistent kernel (chosen per scene by the autotuner).
 struct TraceTuning {
-    uint32_t waves;       // wave64 workgroups launched
+    uint32_t cus;          // compute units of the device
+    uint32_t waves_per_cu; // wave64 workgroups launched per CU, at most as many as it holds
     uint32_t refill_min;  // idle lanes that trigger a refill (1..64)
     uint32_t lds_depth;   // stack entries per lane kept in LDS (8, 16, 24)
     uint32_t occupancy;   // register budget as waves per SIMD (4 or 8)

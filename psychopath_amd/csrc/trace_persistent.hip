@@ -20,6 +20,9 @@
 //     keeps no transform, lerp or nesting state in registers.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
+#include <atomic>
+
 #include "layout.h"
 #include "psymath.h"
 #include "trace.h"
@@ -609,25 +612,56 @@ void trace_persistent_kernel(TraceArgs a, unsigned int* work, uint32_t refill_mi
     }
 }
 
+// Zeroes the ranges' counters with a kernel, so the launch sequence can be
+// captured in a graph (no memset node).
+__global__ void reset_work_kernel(unsigned int* work) { work[threadIdx.x * TRACE_RANGE_WORDS] = 0u; }
+
+// Launches one build of the kernel with at most as many waves as the chip
+// holds at once (its registers and LDS decide; the same on every gfx950, so
+// asked once per build): the waves start on equal shares of the rays, and a
+// wave that has to wait for another to end starts its share that late.
+// Launched at 24 per CU where 20 fit, 16.7M incoherent rays took 3.42 ms and
+// at 20 3.33; the motion scene's 1M rays 1.70 ms at 20 where 16 fit and 1.35
+// at 16.
+template <auto KERNEL>
+hipError_t launch_resident(const TraceArgs& a, unsigned int* work, const TraceTuning& tune, hipStream_t s) {
+    static std::atomic<uint32_t> resident{0};
+    uint32_t per_cu = resident.load(std::memory_order_relaxed);
+    if (per_cu == 0) {
+        int blocks = 0;
+        hipError_t e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&blocks, KERNEL, WAVE, 0);
+        if (e != hipSuccess) return e;
+        per_cu = (uint32_t)std::max(1, blocks);
+        resident.store(per_cu, std::memory_order_relaxed);
+    }
+    const uint32_t waves =
+        (tune.cus * std::min(tune.waves_per_cu, per_cu) + TRACE_RANGES - 1u) / TRACE_RANGES * TRACE_RANGES;
+    // Waves that start on all of the rays read no counter.
+    if (a.n_dev ||
+        (uint64_t)first_rays((uint32_t)a.n, waves) * (waves / TRACE_RANGES) < range_count((uint32_t)a.n, 0)) {
+        hipLaunchKernelGGL(reset_work_kernel, dim3(1), dim3(TRACE_RANGES), 0, s, work);
+        const hipError_t e = hipGetLastError();
+        if (e != hipSuccess) return e;
+    }
+    hipLaunchKernelGGL(KERNEL, dim3(waves), dim3(WAVE), 0, s, a, work, tune.refill_min, tune.leaf_min);
+    return hipGetLastError();
+}
+
 template <bool COUNT, bool XF, bool MOTION, uint32_t RING, bool NESTED, bool BIG>
 hipError_t launch_one(const TraceArgs& a, unsigned int* work, const TraceTuning& tune, hipStream_t s) {
     // Register budget: 8 waves per SIMD caps the kernel at 64 VGPRs (the
     // compiler keeps the rest in private memory), 4 lets it use up to 128.
     // The cooperative node fetch serves static single-level scenes.
-    auto launch = [&](auto kernel) {
-        hipLaunchKernelGGL(kernel, dim3(tune.waves), dim3(WAVE), 0, s, a, work, tune.refill_min, tune.leaf_min);
-        return hipGetLastError();
-    };
     if constexpr (!COUNT && !MOTION && !NESTED) {
         if (tune.coop) {
-            if (tune.occupancy >= 8) return launch(trace_persistent_kernel<false, XF, false, RING, 8, true, false, false>);
-            return launch(trace_persistent_kernel<false, XF, false, RING, 4, true, false, false>);
+            if (tune.occupancy >= 8) return launch_resident<&trace_persistent_kernel<false, XF, false, RING, 8, true, false, false>>(a, work, tune, s);
+            return launch_resident<&trace_persistent_kernel<false, XF, false, RING, 4, true, false, false>>(a, work, tune, s);
         }
     }
     if constexpr (!COUNT && !BIG) {
-        if (tune.occupancy >= 8) return launch(trace_persistent_kernel<false, XF, MOTION, RING, 8, false, NESTED, false>);
+        if (tune.occupancy >= 8) return launch_resident<&trace_persistent_kernel<false, XF, MOTION, RING, 8, false, NESTED, false>>(a, work, tune, s);
     }
-    return launch(trace_persistent_kernel<COUNT, XF, MOTION, RING, 4, false, NESTED, BIG>);
+    return launch_resident<&trace_persistent_kernel<COUNT, XF, MOTION, RING, 4, false, NESTED, BIG>>(a, work, tune, s);
 }
 
 template <bool COUNT, bool XF, bool MOTION, bool NESTED>
@@ -665,25 +699,12 @@ hipError_t launch_feat(const TraceArgs& a, unsigned int* work, const TraceTuning
 
 }  // namespace
 
-// Zeroes the ranges' counters with a kernel, so the launch sequence can be
-// captured in a graph (no memset node).
-__global__ void reset_work_kernel(unsigned int* work) { work[threadIdx.x * TRACE_RANGE_WORDS] = 0u; }
-
 hipError_t launch_trace_persistent(const TraceArgs& args, bool counted, bool has_xf, bool has_motion,
-                                   unsigned int* work, const TraceTuning& tuning, hipStream_t stream) {
+                                   unsigned int* work, const TraceTuning& tune, hipStream_t stream) {
     if (args.n == 0) return hipSuccess;
-    TraceTuning tune = tuning;
-    tune.waves = (tune.waves + TRACE_RANGES - 1u) / TRACE_RANGES * TRACE_RANGES;
-    if (args.n >= 0x80000000ull || tune.waves == 0 || tune.refill_min == 0 || tune.refill_min > 64 ||
-        tune.leaf_min > 64)
+    if (args.n >= 0x80000000ull || tune.cus == 0 || tune.waves_per_cu == 0 || tune.refill_min == 0 ||
+        tune.refill_min > 64 || tune.leaf_min > 64)
         return hipErrorInvalidValue;
-    // A launch whose waves start on all of its rays reads no counter.
-    const uint32_t n = (uint32_t)args.n;
-    if (args.n_dev || (uint64_t)first_rays(n, tune.waves) * (tune.waves / TRACE_RANGES) < range_count(n, 0)) {
-        hipLaunchKernelGGL(reset_work_kernel, dim3(1), dim3(TRACE_RANGES), 0, stream, work);
-        hipError_t e = hipGetLastError();
-        if (e != hipSuccess) return e;
-    }
     return counted ? launch_feat<true>(args, work, tune, has_xf, has_motion, stream)
                    : launch_feat<false>(args, work, tune, has_xf, has_motion, stream);
 }
