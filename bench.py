@@ -348,7 +348,7 @@ RENDER_BYTES = {
     "closest_ray": 57,    # per closest-hit ray: ray in (8 floats) + SoA hit out (kind, t, b0-b2, prim, inst)
     "shadow_ray": 33,     # per shadow ray: ray in + hit kind out
     "instance": 80,       # per instance entry: instance record + one transform
-    "shadow": 53,         # per shadow result: kind, path, colour and pending in, colour out
+    "shadow": 49,         # per shadow result, added by the shading step: kind, pending and colour in, colour out
     "sort": 14,           # per closest hit: kind and instance twice, order out
     "shade": 310,         # per closest hit: path state in/out, hit, ray, triangle and instance records, 2 queued rays
     "film": 68,           # per path: colour and wavelength in, XYZ out and in, film read-modify-write
@@ -366,9 +366,8 @@ def render_roofline(prof: dict, cnt: dict, node_b: int, tri_b: int) -> dict:
                           prof["closest_rays"] * b["closest_ray"]),
         "trace_shadow": (prof["shadow_trace_ms"], cnt["shadow_node_visits"] * node_b + cnt["shadow_tri_tests"] * tri_b +
                          prof["shadow_rays"] * b["shadow_ray"]),
-        "shadow_results": (prof["shadow_ms"], prof["shadow_rays"] * b["shadow"]),
         "sort": (prof["sort_ms"], prof["closest_rays"] * b["sort"]),
-        "shade": (prof["shade_ms"], prof["closest_rays"] * b["shade"]),
+        "shade": (prof["shade_ms"], prof["closest_rays"] * b["shade"] + prof["shadow_rays"] * b["shadow"]),
         "film": (prof["film_ms"], prof["paths"] * b["film"]),
     }
     extra = cnt["instance_visits"] * b["instance"]

@@ -180,8 +180,9 @@ int psy_renderer_set_options(psy_renderer* renderer, uint32_t flags);
  * PSY_RENDER_PROFILE (stage times, paths, rays) and PSY_RENDER_COUNT
  * (traversal counters of closest-hit and shadow rays); the call resets
  * them.  Stage times are device milliseconds between HIP events around each
- * kernel: camera_kernel, the closest-hit and shadow traversals, shadow
- * results, the material sort, shade_kernel, and the film kernels. */
+ * kernel: camera_kernel, the closest-hit and shadow traversals (one launch
+ * in ordinary renders, two here), the material sort, shade_kernel, and the
+ * film kernels; shadow_ms is 0, as the shading step adds shadow results. */
 typedef struct {
     double camera_ms, trace_ms, shadow_trace_ms, shadow_ms, sort_ms, shade_ms, film_ms;
     uint64_t paths, closest_rays, shadow_rays;

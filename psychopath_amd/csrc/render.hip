@@ -8,11 +8,10 @@
 //
 //   camera    Camera::generate_ray + LightPath::new for every path slot
 //   trace     closest-hit queue and shadow queue through the persistent
-//             traversal kernel (counts read on the device)
-//   shadow    unoccluded shadow rays add their pending light
+//             traversal kernel, in one launch (counts read on the device)
 //   sort      closest hits binned by closure kind (miss, light, Lambert,
 //             GGX, emit) so the shading waves run one closure's code
-//   shade     emission / background, next-event estimation through the light
+//   shade     the last shadow ray's light, emission / background, next-event estimation through the light
 //             tree, BSDF sampling; appends the next shadow and bounce rays
 //   film      path colour -> XYZ, added per pixel in sample order
 //
@@ -92,14 +91,6 @@ __device__ __forceinline__ void queue_put(const Queue& q, uint32_t at, uint32_t 
 
 __global__ void wave_begin_kernel(uint32_t* wave_idx, uint32_t value) { *wave_idx = value; }
 __global__ void wave_advance_kernel(uint32_t* wave_idx) { *wave_idx += 1u; }
-
-// Zeroes the closest and shadow output counters and the sort bins.
-__global__ void reset_counts_kernel(uint32_t* a, uint32_t* b, uint32_t* bins) {
-    const int i = threadIdx.x;
-    if (i == 0) *a = 0u;
-    if (i == 1) *b = 0u;
-    if (i < 2 * (int)NUM_BINS) bins[i] = 0u;
-}
 
 __global__ void zero_film_kernel(float* film, uint64_t n) {
     for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (uint64_t)gridDim.x * blockDim.x)
@@ -188,7 +179,7 @@ __device__ __forceinline__ void camera_path(const ShadeScene& sc, const ReqParam
 // Camera::generate_ray and LightPath::new for every slot of the wave.
 __global__ __launch_bounds__(KBLOCK) void camera_kernel(const WavePlan* plans, const uint32_t* wave_idx,
                                                         const ReqParams* reqs, ShadeScene sc, Paths P, Queue qa,
-                                                        uint32_t* shadow_count) {
+                                                        uint32_t* shadow_count, unsigned int* work) {
     const WavePlan& plan = plans[*wave_idx];
     const uint32_t total = plan.total;
     const uint32_t i0 = blockIdx.x * blockDim.x + threadIdx.x;
@@ -196,6 +187,8 @@ __global__ __launch_bounds__(KBLOCK) void camera_kernel(const WavePlan* plans, c
         *qa.count = total;
         *shadow_count = 0u;
     }
+    // the ray counters of the wave's first traversal launch
+    if (i0 < TRACE_RANGES) work[i0 * TRACE_RANGE_WORDS] = 0u;
     for (uint32_t i = i0; i < total; i += gridDim.x * blockDim.x) {
         const WaveSeg& sg = find_seg(plan, i);
         const ReqParams rp = reqs[sg.req];
@@ -207,6 +200,7 @@ __global__ __launch_bounds__(KBLOCK) void camera_kernel(const WavePlan* plans, c
         P.sample[i] = ps.sample;
         P.seed[i] = ps.seed;
         P.bounces[i] = 0u;
+        P.shadow[i] = PSY_HIT_OCCLUDE;
         P.wl[i] = ps.wl;
         P.time[i] = ps.time;
         P.csp[i] = 1.0f;
@@ -215,19 +209,6 @@ __global__ __launch_bounds__(KBLOCK) void camera_kernel(const WavePlan* plans, c
         s4_store(P.pending, i, ps.pending);
         P.has_next[i] = 0u;
         queue_put(qa, i, i, o, d, ps.time, __builtin_huge_valf());
-    }
-}
-
-// Shadow-ray results (renderer.rs:670-690): a miss adds the pending light.
-__global__ __launch_bounds__(KBLOCK) void shadow_kernel(Queue qs, const uint8_t* kind, Paths P,
-                                                        unsigned long long* rays) {
-    const uint32_t n = *qs.count;
-    if (blockIdx.x == 0 && threadIdx.x == 0) atomicAdd(rays, (unsigned long long)n);
-    for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) {
-        if (kind[i] != PSY_HIT_MISS) continue;
-        const uint32_t p = qs.path[i];
-        const S4 c = s4_load(P.color, p) + s4_load(P.pending, p);
-        s4_store(P.color, p, c);
     }
 }
 
@@ -739,7 +720,6 @@ __global__ __launch_bounds__(KBLOCK) __attribute__((amdgpu_waves_per_eu(MINW))) 
     ShadeScene sc, const ReqParams* reqs, Paths P, Queue qa, Hits h, const uint32_t* order, Queue qa_out,
     Queue qs_out) {
     const uint32_t n = *qa.count;
-    if (blockIdx.x == 0 && threadIdx.x == 0) atomicAdd(sc.rays, (unsigned long long)n);
     const uint32_t stride = gridDim.x * blockDim.x;
     // Every thread of a block runs the loop the same number of times, so the
     // block-wide appends see all of them.  One atomic per block and queue:
@@ -776,7 +756,16 @@ __global__ __launch_bounds__(KBLOCK) __attribute__((amdgpu_waves_per_eu(MINW))) 
             ptime = ps.time;
             const HitRec hr{h.kind[q], h.t[q], h.b0[q], h.b1[q], h.b2[q], h.prim[q], h.inst[q]};
             shade_path<true>(sc, rp, ps, hr, v3(qa.ox[q], qa.oy[q], qa.oz[q]), v3(qa.dx[q], qa.dy[q], qa.dz[q]), so);
-            if (so.added) s4_store(P.color, p, s4_load(P.color, p) + so.add);
+            // The last shadow ray's light (renderer.rs:670-690), then what
+            // this event adds.
+            const bool lit = P.shadow[p] == PSY_HIT_MISS;
+            if (lit || so.added) {
+                S4 c = s4_load(P.color, p);
+                if (lit) c = c + s4_load(P.pending, p);
+                if (so.added) c = c + so.add;
+                s4_store(P.color, p, c);
+            }
+            if (lit) P.shadow[p] = PSY_HIT_OCCLUDE;
             if (so.kept) {
                 const float4 a = P.next_o[p], b = P.next_d[p];
                 so.bo = v3(a.x, a.y, a.z);
@@ -895,12 +884,15 @@ __global__ __launch_bounds__(MEGA_BLOCK) __attribute__((amdgpu_waves_per_eu(MINW
     px[2] = fz;
 }
 
-// Path colour to XYZ (XYZ::from_spectral_sample, color.rs:520-526), one
-// lane per slot; the result replaces the slot's colour.
+// Path colour, with the light of a last shadow ray that no shading step
+// followed, to XYZ (XYZ::from_spectral_sample, color.rs:520-526), one lane per
+// slot; the result replaces the slot's colour.
 __global__ __launch_bounds__(KBLOCK) void xyz_kernel(const WavePlan* plans, const uint32_t* wave_idx, Paths P) {
     const uint32_t total = plans[*wave_idx].total;
     for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < total; i += gridDim.x * blockDim.x) {
-        const V3 c = xyz_from_spectral(s4_load(P.color, i), P.wl[i]);
+        S4 sum = s4_load(P.color, i);
+        if (P.shadow[i] == PSY_HIT_MISS) sum = sum + s4_load(P.pending, i);
+        const V3 c = xyz_from_spectral(sum, P.wl[i]);
         P.color[i] = make_float4(c.x, c.y, c.z, 0.0f);
     }
 }
@@ -1058,23 +1050,33 @@ uint32_t grid_for(uint64_t n) { return (uint32_t)std::max<uint64_t>(1, std::min<
 
 namespace {
 
-TraceArgs queue_args(const psy_renderer* r, const Queue& q, const Hits& h, bool occlusion) {
+// Traversal of a step's closest-hit queue `qa`, its shadow queue `qs`, or
+// both in one launch.
+TraceArgs queue_args(const psy_renderer* r, const Queue& qa, const Queue& qs, bool closest, bool shadow) {
     TraceArgs a = scene_args(r->scene);
-    a.ox = q.ox; a.oy = q.oy; a.oz = q.oz;
-    a.dx = q.dx; a.dy = q.dy; a.dz = q.dz;
-    a.time = q.time; a.max_t = q.max_t;
-    a.flags = nullptr;
-    a.all_occlusion = occlusion ? 1u : 0u;
-    a.n = r->capacity;
-    a.n_dev = q.count;
-    a.kind = h.kind;
-    a.t = h.t; a.b0 = h.b0; a.b1 = h.b1; a.b2 = h.b2;
-    a.prim_id = h.prim; a.inst_id = h.inst;
+    a.ox = qa.ox; a.oy = qa.oy; a.oz = qa.oz;
+    a.dx = qa.dx; a.dy = qa.dy; a.dz = qa.dz;
+    a.time = qa.time; a.max_t = qa.max_t;
+    if (closest) {
+        a.n = r->capacity;
+        a.n_dev = qa.count;
+        const Hits& h = r->ha;
+        a.kind = h.kind;
+        a.t = h.t; a.b0 = h.b0; a.b1 = h.b1; a.b2 = h.b2;
+        a.prim_id = h.prim; a.inst_id = h.inst;
+    }
+    if (shadow) {
+        a.n2_dev = qs.count;
+        a.n2_at = (uint32_t)r->capacity;
+        a.n2_out = qa.path;
+        a.n2_kind = r->P.shadow;
+    }
+    a.tally = r->sc.rays;
     return a;
 }
 
 // Stages of the renderer's profile (psy_render_profile).
-enum { ST_CAMERA, ST_TRACE, ST_SHADOW_TRACE, ST_SHADOW, ST_SORT, ST_SHADE, ST_FILM };
+enum { ST_CAMERA, ST_TRACE, ST_SHADOW_TRACE, ST_SORT, ST_SHADE, ST_FILM, ST_COUNT };
 
 // Adds a device queue count to a 64-bit tally (profile mode).
 __global__ void accum_count_kernel(const uint32_t* count, unsigned long long* acc) { *acc += *count; }
@@ -1106,51 +1108,69 @@ int staged(psy_renderer* r, int stage, F&& launch) {
     return PSY_OK;
 }
 
-// Enqueues the steps of one wave: camera, `steps` closest/shadow rounds, the
-// last shadow round and the film.  The wave's plan is plans[*wave_idx].
+// Enqueues the steps of one wave: camera, `steps` rounds of traversal and
+// shading, the last shadow rays and the film.  The wave's plan is
+// plans[*wave_idx].  A step's closest-hit and shadow rays are one launch, so
+// their last, longest rays overlap: the late steps of a wave trace few rays
+// and take as long as those do.  Traced one after the other, with the shadow
+// results added by a kernel and the counters zeroed by three, the motion
+// scene took 16.3 ms at 960x540 and 4 spp (13.6 now), the large scene 12.5 ms
+// at full HD and 2 spp (10.1), the Cornell box 0.72 ms at 64x64 (0.60).  With profiling or counting they are two, so
+// each can be timed and counted.
 int enqueue_wave(psy_renderer* r, uint32_t steps) {
     const hipStream_t s = r->stream;
     const uint32_t grid = grid_for(r->capacity);
     const bool tally = r->profile || r->counted;
     Queue qa_in = r->qa[0], qa_out = r->qa[1], qs_in = r->qs[0], qs_out = r->qs[1];
+    unsigned int *work = r->work, *work_next = r->work + TRACE_WORK_WORDS;
     int rc = staged(r, ST_CAMERA, [&]() -> int {
         hipLaunchKernelGGL(camera_kernel, dim3(grid), dim3(KBLOCK), 0, s, r->plans, r->wave_idx, r->reqs, r->sc, r->P,
-                           qa_in, qs_in.count);
+                           qa_in, qs_in.count, work);
         PSY_HIP(hipGetLastError());
         return PSY_OK;
     });
     if (rc) return rc;
     psy_trace_tuning tune = r->tuning;
     if (tune.kernel == PSY_KERNEL_SIMPLE) tune.kernel = PSY_KERNEL_PERSISTENT;
-    auto trace = [&](const Queue& q, const Hits& h, bool occl, unsigned int* work, int stage) -> int {
-        TraceArgs a = queue_args(r, q, h, occl);
-        a.counters = r->prof_dev + (occl ? 7 : 2);
-        int e2 = staged(r, stage, [&]() -> int {
+    auto trace = [&](TraceArgs a, int stage) -> int {
+        a.counters = r->prof_dev + (stage == ST_TRACE ? 2 : 7);
+        return staged(r, stage, [&]() -> int {
             hipError_t e = launch_tuned(r->scene, tune, r->cu_count, work, a, r->counted, s);
             if (e != hipSuccess) return fail(PSY_E_DEVICE, std::string("trace launch: ") + hipGetErrorString(e));
             return PSY_OK;
         });
-        if (e2 || !tally) return e2;
-        hipLaunchKernelGGL(accum_count_kernel, dim3(1), dim3(1), 0, s, q.count, r->prof_dev + (occl ? 1 : 0));
-        PSY_HIP(hipGetLastError());
-        return PSY_OK;
     };
     for (uint32_t step = 0; step <= steps; step++) {
         const bool last = step == steps;
-        if (!last) {
-            rc = trace(qa_in, r->ha, false, r->work, ST_TRACE);
+        // The first traversal launch of a step also zeroes the counts that
+        // its sorting and shading add to.
+        auto clears = [&](TraceArgs a) {
+            if (last) return a;
+            a.clear0 = qa_out.count;
+            a.clear1 = qs_out.count;
+            a.clear_run = r->counts + COUNTS_BINS;
+            a.clear_run_n = 2 * NUM_BINS;
+            return a;
+        };
+        if (!tally) {
+            TraceArgs a = clears(queue_args(r, qa_in, qs_in, !last, true));
+            a.work_next = work_next;
+            rc = trace(a, ST_TRACE);
             if (rc) return rc;
-        }
-        rc = trace(qs_in, r->hs, true, r->work + TRACE_WORK_WORDS, ST_SHADOW_TRACE);
-        if (!rc) rc = staged(r, ST_SHADOW, [&]() -> int {
-            hipLaunchKernelGGL(shadow_kernel, dim3(grid), dim3(KBLOCK), 0, s, qs_in, r->hs.kind, r->P, r->sc.rays);
+            std::swap(work, work_next);
+        } else {
+            if (!last) {
+                rc = trace(clears(queue_args(r, qa_in, qs_in, true, false)), ST_TRACE);
+                if (rc) return rc;
+                hipLaunchKernelGGL(accum_count_kernel, dim3(1), dim3(1), 0, s, qa_in.count, r->prof_dev);
+                PSY_HIP(hipGetLastError());
+            }
+            rc = trace(queue_args(r, qa_in, qs_in, false, true), ST_SHADOW_TRACE);
+            if (rc) return rc;
+            hipLaunchKernelGGL(accum_count_kernel, dim3(1), dim3(1), 0, s, qs_in.count, r->prof_dev + 1);
             PSY_HIP(hipGetLastError());
-            return PSY_OK;
-        });
-        if (rc) return rc;
+        }
         if (last) break;
-        hipLaunchKernelGGL(reset_counts_kernel, dim3(1), dim3(64), 0, s, qa_out.count, qs_out.count, r->counts + COUNTS_BINS);
-        PSY_HIP(hipGetLastError());
         const uint32_t* order = nullptr;
         if (r->sort_materials) {
             rc = staged(r, ST_SORT, [&]() -> int {
@@ -1425,6 +1445,7 @@ int psy_renderer_create(const psy_scene* scene_c, const psy_world_desc* world, u
     if (!rc) rc = r->alloc(&P.sample, C);
     if (!rc) rc = r->alloc(&P.seed, C);
     if (!rc) rc = r->alloc(&P.bounces, C);
+    if (!rc) rc = r->alloc(&P.shadow, C);
     if (!rc) rc = r->alloc(&P.wl, C);
     if (!rc) rc = r->alloc(&P.time, C);
     if (!rc) rc = r->alloc(&P.csp, C);
@@ -1435,18 +1456,12 @@ int psy_renderer_create(const psy_scene* scene_c, const psy_world_desc* world, u
     if (!rc) rc = r->alloc(&P.next_o, C);
     if (!rc) rc = r->alloc(&P.next_d, C);
     if (!rc) rc = r->alloc(&P.next_fac, C);
-    for (int k = 0; k < 2 && !rc; k++) rc = r->alloc_queue(r->qa[k]);
-    for (int k = 0; k < 2 && !rc; k++) rc = r->alloc_queue(r->qs[k]);
+    for (int k = 0; k < 2 && !rc; k++) rc = r->alloc_queues(r->qa[k], r->qs[k]);
     if (!rc) rc = r->alloc(&r->ha.kind, C);
     float** hf[4] = {&r->ha.t, &r->ha.b0, &r->ha.b1, &r->ha.b2};
     for (int k = 0; k < 4 && !rc; k++) rc = r->alloc(hf[k], C);
     if (!rc) rc = r->alloc(&r->ha.prim, C);
     if (!rc) rc = r->alloc(&r->ha.inst, C);
-    if (!rc) rc = r->alloc(&r->hs.kind, C);
-    float** sf[4] = {&r->hs.t, &r->hs.b0, &r->hs.b1, &r->hs.b2};
-    for (int k = 0; k < 4 && !rc; k++) rc = r->alloc(sf[k], C);
-    if (!rc) rc = r->alloc(&r->hs.prim, C);
-    if (!rc) rc = r->alloc(&r->hs.inst, C);
     if (!rc) rc = r->alloc(&r->order, C);
     if (!rc) rc = r->alloc(&r->counts, COUNTS_WORDS);
     if (!rc) rc = r->alloc(&r->wave_idx, 1);
@@ -1656,9 +1671,8 @@ int psy_renderer_get_profile(psy_renderer* r, psy_render_profile* p) {
     PSY_HIP(hipMemcpy(c, r->prof_dev, sizeof(c), hipMemcpyDeviceToHost));
     PSY_HIP(hipMemset(r->prof_dev, 0, sizeof(c)));
     std::memset(p, 0, sizeof(*p));
-    double* ms[7] = {&p->camera_ms, &p->trace_ms, &p->shadow_trace_ms, &p->shadow_ms, &p->sort_ms, &p->shade_ms,
-                     &p->film_ms};
-    for (int i = 0; i < 7; i++) {
+    double* ms[ST_COUNT] = {&p->camera_ms, &p->trace_ms, &p->shadow_trace_ms, &p->sort_ms, &p->shade_ms, &p->film_ms};
+    for (int i = 0; i < ST_COUNT; i++) {
         *ms[i] = r->stage_ms[i];
         r->stage_ms[i] = 0.0;
     }

@@ -114,6 +114,11 @@ struct Paths {
     uint32_t* sample;
     uint32_t* seed;
     uint32_t* bounces;
+    // The path's shadow ray: PSY_HIT_MISS when the last one reached its light,
+    // so the pending contribution is due; PSY_HIT_OCCLUDE when it did not or
+    // there was none.  The traversal writes it, the next shading step or the
+    // film adds the contribution.
+    uint8_t* shadow;
     float* wl;
     float* time;
     float* csp;  // closure_sample_pdf
@@ -181,7 +186,7 @@ struct psy_renderer {
         hipEvent_t a, b;
     };
     std::vector<Mark> marks;
-    double stage_ms[7] = {};
+    double stage_ms[6] = {};  // by stage (render.hip)
     uint64_t prof_paths = 0;
     unsigned long long* prof_dev = nullptr;
 
@@ -189,7 +194,7 @@ struct psy_renderer {
     ShadeScene sc{};
     Paths P{};
     Queue qa[2]{}, qs[2]{};
-    Hits ha{}, hs{};
+    Hits ha{};  // of the closest-hit queue
     uint32_t* order = nullptr;
     uint32_t* counts = nullptr;  // COUNTS_WORDS words: queue counts, sort bins, rays traced (u64)
     uint32_t* wave_idx = nullptr;
@@ -243,10 +248,17 @@ struct psy_renderer {
             }
     }
 
-    int alloc_queue(Queue& q) {
-        int r = alloc(&q.path, capacity);
-        float** f[8] = {&q.ox, &q.oy, &q.oz, &q.dx, &q.dy, &q.dz, &q.time, &q.max_t};
-        for (int k = 0; k < 8 && !r; k++) r = alloc(f[k], capacity);
+    // The closest-hit queue `a` and the shadow queue `s` of one step, halves
+    // of the same arrays: one launch traces both.
+    int alloc_queues(Queue& a, Queue& s) {
+        int r = alloc(&a.path, 2 * capacity);
+        if (!r) s.path = a.path + capacity;
+        float** fa[8] = {&a.ox, &a.oy, &a.oz, &a.dx, &a.dy, &a.dz, &a.time, &a.max_t};
+        float** fs[8] = {&s.ox, &s.oy, &s.oz, &s.dx, &s.dy, &s.dz, &s.time, &s.max_t};
+        for (int k = 0; k < 8 && !r; k++) {
+            r = alloc(fa[k], 2 * capacity);
+            if (!r) *fs[k] = *fa[k] + capacity;
+        }
         return r;
     }
 };

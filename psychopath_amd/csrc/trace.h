@@ -45,6 +45,22 @@ struct TraceArgs {
     uint32_t all_occlusion;    // every ray is an occlusion ray (flags ignored)
     uint64_t n;                // ray count, or the capacity when n_dev is set
     const uint32_t* n_dev;     // device-resident ray count (persistent kernel), or NULL
+    // Persistent kernels: occlusion rays traced in the same launch after the
+    // n rays above (counted by n2_dev; NULL: none), at index n2_at of the
+    // same ray arrays.  Ray i's result is the kind byte n2_kind[n2_out[i]].
+    const uint32_t* n2_dev;
+    uint32_t n2_at;
+    const uint32_t* n2_out;
+    uint8_t* n2_kind;
+    // Persistent kernels, for a caller that launches one after another: the
+    // first block zeroes clear0[0], clear1[0] and clear_run[0, clear_run_n)
+    // where not NULL, adds the rays to *tally, and when `work_next` is set
+    // zeroes those counters, which the next launch then takes without a
+    // reset of its own (so must this launch's `work` be clear).
+    uint32_t *clear0, *clear1, *clear_run;
+    uint32_t clear_run_n;
+    unsigned long long* tally;
+    unsigned int* work_next;
     // hits (device): 32-byte records when `rec` is set, else structure of
     // arrays
     uint4* rec;

@@ -138,7 +138,18 @@ void trace_persistent_kernel(TraceArgs a, unsigned int* work, uint32_t refill_mi
     uint32_t spill[TRACE_STACK_CAPACITY];
     uint32_t sp = 0, bot = 0;
 
-    const uint32_t n = a.n_dev ? *a.n_dev : (uint32_t)a.n;
+    // Rays [0, n1) stand at their own index, [n1, n) are the second set's.
+    const uint32_t n1 = a.n_dev ? *a.n_dev : (uint32_t)a.n;
+    const uint32_t n = n1 + (a.n2_dev ? *a.n2_dev : 0u);
+    if (blockIdx.x == 0) {
+        if (a.work_next && lane < (int)TRACE_RANGES) a.work_next[lane * TRACE_RANGE_WORDS] = 0u;
+        if (a.clear_run && lane < (int)a.clear_run_n) a.clear_run[lane] = 0u;
+        if (lane == 0) {
+            if (a.clear0) *a.clear0 = 0u;
+            if (a.clear1) *a.clear1 = 0u;
+            if (a.tally) atomicAdd(a.tally, (unsigned long long)n);
+        }
+    }
     const Xf ident = xf_identity();
 
     // Per-lane ray state.
@@ -232,11 +243,14 @@ void trace_persistent_kernel(TraceArgs a, unsigned int* work, uint32_t refill_mi
                 if (rank < avail) {
                     has = true;
                     ray = range_ray(rx, next + rank);
+                    const bool second = ray >= n1;
+                    if (second) ray = ray - n1 + a.n2_at;
                     o = v3(a.ox[ray], a.oy[ray], a.oz[ray]);
                     d = v3(a.dx[ray], a.dy[ray], a.dz[ray]);
                     time = MOTION || XF ? a.time[ray] : 0.0f;
                     tmax = a.max_t[ray];
-                    occl = a.all_occlusion != 0 || (a.flags != nullptr && (a.flags[ray] & 1u) != 0);
+                    occl = second || a.all_occlusion != 0 || (a.flags != nullptr && (a.flags[ray] & 1u) != 0);
+                    if (second) ray = a.n2_out[ray];  // (from here on only the result's place)
                     // Top-level local ray: update_local with the identity
                     // (tracer.rs:65-70).
                     lo = xf_point(ident, o);
@@ -579,7 +593,9 @@ void trace_persistent_kernel(TraceArgs a, unsigned int* work, uint32_t refill_mi
         }
 
         if (finished) {
-            if (a.rec != nullptr) {
+            if (a.n2_kind != nullptr && occl) {
+                a.n2_kind[ray] = kind;
+            } else if (a.rec != nullptr) {
                 // One 32-byte record per ray, two 16-byte stores: rays finish
                 // out of order, and a whole record fills a memory sector
                 // where the seven arrays of the SoA form leave seven partial
@@ -637,8 +653,8 @@ hipError_t launch_resident(const TraceArgs& a, unsigned int* work, const TraceTu
     const uint32_t waves =
         (tune.cus * std::min(tune.waves_per_cu, per_cu) + TRACE_RANGES - 1u) / TRACE_RANGES * TRACE_RANGES;
     // Waves that start on all of the rays read no counter.
-    if (a.n_dev ||
-        (uint64_t)first_rays((uint32_t)a.n, waves) * (waves / TRACE_RANGES) < range_count((uint32_t)a.n, 0)) {
+    if (!a.work_next && (a.n_dev || a.n2_dev ||
+        (uint64_t)first_rays((uint32_t)a.n, waves) * (waves / TRACE_RANGES) < range_count((uint32_t)a.n, 0))) {
         hipLaunchKernelGGL(reset_work_kernel, dim3(1), dim3(TRACE_RANGES), 0, s, work);
         const hipError_t e = hipGetLastError();
         if (e != hipSuccess) return e;
@@ -701,7 +717,7 @@ hipError_t launch_feat(const TraceArgs& a, unsigned int* work, const TraceTuning
 
 hipError_t launch_trace_persistent(const TraceArgs& args, bool counted, bool has_xf, bool has_motion,
                                    unsigned int* work, const TraceTuning& tune, hipStream_t stream) {
-    if (args.n == 0) return hipSuccess;
+    if (args.n == 0 && !args.n2_dev) return hipSuccess;
     if (args.n >= 0x80000000ull || tune.cus == 0 || tune.waves_per_cu == 0 || tune.refill_min == 0 ||
         tune.refill_min > 64 || tune.leaf_min > 64)
         return hipErrorInvalidValue;
