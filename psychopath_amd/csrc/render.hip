@@ -728,9 +728,10 @@ __global__ __launch_bounds__(KBLOCK) __attribute__((amdgpu_waves_per_eu(MINW))) 
     __shared__ uint32_t app_cnt[2 * (KBLOCK / 64)], app_base[2 * (KBLOCK / 64)];
     const uint32_t n_round = (n + (uint32_t)KBLOCK - 1u) / (uint32_t)KBLOCK * (uint32_t)KBLOCK;
     for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < n_round; i += stride) {
-        ShadeOut so;
-        so.shadow = false;
-        so.bounce = false;
+        // Every field starts defined: with those a path does not use left
+        // undefined, the build for 3 waves per SIMD lost the emission of
+        // light hits.
+        ShadeOut so{};
         float ptime = 0.0f;
         uint32_t p = 0;
         if (i < n) {
@@ -836,7 +837,7 @@ __global__ __launch_bounds__(MEGA_BLOCK) __attribute__((amdgpu_waves_per_eu(MINW
                 const TraceHit th = trace_one<false, MEGA_LDS, MEGA_SPILL, true>(ta, o, d, ps.time, __builtin_huge_valf(),
                                                                            false, lds_col, MEGA_BLOCK, tc);
                 const HitRec hr{th.kind, th.t, th.b0, th.b1, th.b2, th.prim, th.inst};
-                ShadeOut so;
+                ShadeOut so{};
                 shade_path<false>(sc, rp, ps, hr, o, d, so);
                 traced += so.shadow ? 2u : 1u;
                 if (so.shadow) {
