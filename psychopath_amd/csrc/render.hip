@@ -92,6 +92,17 @@ __device__ __forceinline__ void queue_put(const Queue& q, uint32_t at, uint32_t 
 __global__ void wave_begin_kernel(uint32_t* wave_idx, uint32_t value) { *wave_idx = value; }
 __global__ void wave_advance_kernel(uint32_t* wave_idx) { *wave_idx += 1u; }
 
+// Lays out colours for spectrum_prepared, one block each.
+__global__ void prepare_colors_kernel(const GpuColor* colors, PreparedColor* out) {
+    const GpuColor c = colors[blockIdx.x];
+    PreparedColor& p = out[blockIdx.x];
+    MengCell m{};
+    if (c.kind == PSY_COLOR_XYZ) m = meng_cell(c.a, c.b, c.c);
+    if (threadIdx.x == 0) p.cell = m;
+    for (uint32_t s = threadIdx.x; s < (uint32_t)psy_meng::NUM_SAMPLES; s += blockDim.x)
+        for (int j = 0; j < 4; j++) p.spectrum[s][j] = j < m.n ? psy_meng::POINT_SPECTRUM[m.point[j]][s] : 0.0f;
+}
+
 __global__ void zero_film_kernel(float* film, uint64_t n) {
     for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (uint64_t)gridDim.x * blockDim.x)
         film[i] = 0.0f;
@@ -547,11 +558,20 @@ __device__ __forceinline__ LightPick sample_lights(const ShadeScene& sc, float n
     } else if (lf.top_count) {
         xform = light_xf_at(sc.lxforms + lf.top_start, lf.top_count, time);
     }
-    const LightSample s = inst.kind == PSY_OBJECT_RECT_LIGHT
-                              ? rect_sample_from_point(rect_at(sc.rects[inst.mesh], sc.light_samples, time), xform,
-                                                       is.pos, u, v, wl)
-                              : sphere_sample_from_point(sphere_at(sc.spheres[inst.mesh], sc.light_samples, time),
-                                                         xform, is.pos, u, v, wl);
+    // A light's colour without time samples may be laid out already.
+    auto prepared = [&](auto light, uint32_t at, bool any) {
+        if (any && light.color.kind == PSY_COLOR_XYZ && (light.counts >> 8) == 0u)
+            light.color = prepared_ref(sc.light_colors + at);
+        return light;
+    };
+    const bool rect = inst.kind == PSY_OBJECT_RECT_LIGHT;
+    const LightSample s =
+        rect ? rect_sample_from_point(
+                   prepared(rect_at(sc.rects[inst.mesh], sc.light_samples, time), inst.mesh, inst.mesh < sc.rect_prepared),
+                   xform, is.pos, u, v, wl)
+             : sphere_sample_from_point(prepared(sphere_at(sc.spheres[inst.mesh], sc.light_samples, time),
+                                                 sc.rect_prepared + inst.mesh, inst.mesh < sc.sphere_prepared),
+                                        xform, is.pos, u, v, wl);
     out.found = true;
     out.distant = false;
     out.color = s.color;
@@ -1520,6 +1540,37 @@ int psy_renderer_create(const psy_scene* scene_c, const psy_world_desc* world, u
     std::vector<HaltonDim> hdims;
     std::vector<uint16_t> hperms;
     halton_tables(hdims, hperms);
+    // The colours that shading evaluates again and again, laid out once:
+    // the shaders', the background, and lights' without time samples.
+    {
+        std::vector<GpuColor> colors;
+        for (const GpuClosure& c : shaders) colors.push_back(c.color);
+        colors.push_back(sc.background);
+        const uint32_t fixed = (uint32_t)colors.size();
+        const std::vector<GpuRectLight>& rl = scene->host.rect_lights;
+        const std::vector<GpuSphereLight>& sl = scene->host.sphere_lights;
+        sc.rect_prepared = (uint32_t)std::min<size_t>(rl.size(), PREPARED_LIGHTS);
+        sc.sphere_prepared = (uint32_t)std::min<size_t>(sl.size(), PREPARED_LIGHTS - sc.rect_prepared);
+        for (uint32_t i = 0; i < sc.rect_prepared; i++) colors.push_back(rl[i].color);
+        for (uint32_t i = 0; i < sc.sphere_prepared; i++) colors.push_back(sl[i].color);
+        GpuColor* dcol = nullptr;
+        PreparedColor* prep = nullptr;
+        rc = r->alloc(&prep, colors.size());
+        if (!rc) rc = r->alloc(&dcol, colors.size());
+        if (rc) return bail(rc);
+        e = hipMemcpy(dcol, colors.data(), colors.size() * sizeof(GpuColor), hipMemcpyHostToDevice);
+        if (e == hipSuccess) {
+            hipLaunchKernelGGL(prepare_colors_kernel, dim3((unsigned)colors.size()), dim3(64), 0, r->stream, dcol, prep);
+            e = hipGetLastError();
+        }
+        if (e == hipSuccess) e = hipStreamSynchronize(r->stream);
+        if (e != hipSuccess) return bail(fail(PSY_E_DEVICE, std::string("colour set-up: ") + hipGetErrorString(e)));
+        r->release(dcol);
+        sc.light_colors = prep + fixed;
+        for (size_t i = 0; i < shaders.size(); i++)
+            if (shaders[i].color.kind == PSY_COLOR_XYZ) shaders[i].color = prepared_ref(prep + i);
+        if (sc.background.kind == PSY_COLOR_XYZ) sc.background = prepared_ref(prep + shaders.size());
+    }
     rc = r->alloc(&dsh, shaders.size());
     if (!rc) rc = r->alloc(&ddl, distant.size());
     if (!rc) rc = r->alloc(&dls, distant_samples.size());

@@ -12,6 +12,7 @@
 #pragma once
 
 #include <math.h>
+#include <stddef.h>
 #include <stdint.h>
 
 #include "../../include/psy_render.h"
@@ -416,85 +417,145 @@ RD float nth_wavelength(float hero, int n) {
 // Meng et al.'s upsampling (sub_crates/spectral_upsampling/src/meng.rs:
 // 177-328): xy -> uv grid cell, then bilinear (inside cells) or barycentric
 // (border cells) interpolation of tabulated spectra at four wavelengths.
-RD S4 spectrum_xyz_to_p_4(S4 lambdas, float x, float y, float z) {
+//
+// What depends on the colour alone: the tabulated points in the order their
+// weighted spectra are added, n of them (0: the spectrum is zero).
+struct MengCell {
+    int n;
+    int point[4];
+    float w[4];
+    float inv_norm;
+};
+RD MengCell meng_cell(float x, float y, float z) {
     using namespace psy_meng;
+    MengCell m{};
     float inv_norm = (x + y) + z;
+    m.inv_norm = inv_norm;
     float norm = 1.0f / inv_norm;
-    if (!(norm < 3.40282347e+38f)) return s4_zero();
+    if (!(norm < 3.40282347e+38f)) return m;
     float xx = x * norm, yy = y * norm;
     float u = ((MAT_XY_TO_UV[0] * xx) + (MAT_XY_TO_UV[1] * yy)) + MAT_XY_TO_UV[2];
     float v = ((MAT_XY_TO_UV[3] * xx) + (MAT_XY_TO_UV[4] * yy)) + MAT_XY_TO_UV[5];
-    if (u < 0.0f || u >= (float)GRID_WIDTH || v < 0.0f || v >= (float)GRID_HEIGHT) return s4_zero();
+    if (u < 0.0f || u >= (float)GRID_WIDTH || v < 0.0f || v >= (float)GRID_HEIGHT) return m;
     const int ui = (int)u, vi = (int)v;
     const int* cell = GRID[ui + GRID_WIDTH * vi];
     const bool inside = cell[0] != 0;
     const int num = cell[1];
     const int* idx = cell + 2;
-    if (num == 0) return s4_zero();
-
-    S4 sb;
-    int sb0[4], sb1[4];
-    for (int k = 0; k < 4; k++) {
-        sb.v[k] = ((lambdas.v[k] - SAMPLE_MIN) / (SAMPLE_MAX - SAMPLE_MIN)) * ((float)NUM_SAMPLES - 1.0f);
-        sb0[k] = (int)sb.v[k];
-        sb1[k] = sb0[k] + 1 < NUM_SAMPLES - 1 ? sb0[k] + 1 : NUM_SAMPLES - 1;
-    }
-    S4 sbf = sb - s4((float)sb0[0], (float)sb0[1], (float)sb0[2], (float)sb0[3]);
-    // A cell has at most six points; the loops are unrolled so the points
-    // are indexed by constants and stay in registers.
-    S4 p[6];
-#pragma unroll
-    for (int i = 0; i < 6; i++) {
-        p[i] = s4_zero();
-        if (i < num) {
-            const float* spectrum = POINT_SPECTRUM[idx[i]];
-            S4 p0 = s4(spectrum[sb0[0]], spectrum[sb0[1]], spectrum[sb0[2]], spectrum[sb0[3]]);
-            S4 p1 = s4(spectrum[sb1[0]], spectrum[sb1[1]], spectrum[sb1[2]], spectrum[sb1[3]]);
-            p[i] = (p0 * (s4_splat(1.0f) - sbf)) + (p1 * sbf);
-        }
-    }
-    S4 interp = s4_zero();
+    if (num == 0) return m;
     if (inside) {
         float u2 = u - (float)ui, v2 = v - (float)vi;
-        interp = (((p[0] * ((1.0f - u2) * (1.0f - v2))) + (p[2] * ((1.0f - u2) * v2))) + (p[3] * (u2 * v2))) +
-                 (p[1] * (u2 * (1.0f - v2)));
-    } else {
-        float ex = u - POINT_UV[idx[0]][0];
-        float ey = v - POINT_UV[idx[0]][1];
-        float e0x = POINT_UV[idx[1]][0] - POINT_UV[idx[0]][0];
-        float e0y = POINT_UV[idx[1]][1] - POINT_UV[idx[0]][1];
-        float uu = (e0x * ey) - (ex * e0y);
-        bool found = false;
-#pragma unroll
-        for (int i = 0; i < 5; i++) {
-            if (found || i >= num - 1) continue;
-            float e1x, e1y;
-            if (i == num - 2) {
-                e1x = POINT_UV[idx[1]][0] - POINT_UV[idx[0]][0];
-                e1y = POINT_UV[idx[1]][1] - POINT_UV[idx[0]][1];
-            } else {
-                e1x = POINT_UV[idx[i + 2]][0] - POINT_UV[idx[0]][0];
-                e1y = POINT_UV[idx[i + 2]][1] - POINT_UV[idx[0]][1];
-            }
-            float vv = (ex * e1y) - (e1x * ey);
-            float area = (e0x * e1y) - (e1x * e0y);
-            float uf = uu / area;
-            float vf = vv / area;
-            float wf = (1.0f - uf) - vf;
-            if (uf < 0.0f || vf < 0.0f || wf < 0.0f) {
-                uu = -vv;
-                e0x = e1x;
-                e0y = e1y;
-                continue;
-            }
-            // i + 2 < num here unless i == num - 2, so the clamp never binds.
-            const S4 pc = i == num - 2 ? p[1] : p[i + 2 < 6 ? i + 2 : 5];
-            interp = ((p[0] * wf) + (p[i + 1] * vf)) + (pc * uf);
-            found = true;
-        }
+        m.n = 4;
+        m.point[0] = idx[0]; m.w[0] = (1.0f - u2) * (1.0f - v2);
+        m.point[1] = idx[2]; m.w[1] = (1.0f - u2) * v2;
+        m.point[2] = idx[3]; m.w[2] = u2 * v2;
+        m.point[3] = idx[1]; m.w[3] = u2 * (1.0f - v2);
+        return m;
     }
-    return interp * inv_norm;
+    m.n = 3;  // with weights 0 if no triangle of the border cell holds (u, v)
+    m.point[0] = m.point[1] = m.point[2] = idx[0];
+    float ex = u - POINT_UV[idx[0]][0];
+    float ey = v - POINT_UV[idx[0]][1];
+    float e0x = POINT_UV[idx[1]][0] - POINT_UV[idx[0]][0];
+    float e0y = POINT_UV[idx[1]][1] - POINT_UV[idx[0]][1];
+    float uu = (e0x * ey) - (ex * e0y);
+    for (int i = 0; i < num - 1; i++) {
+        const int next = i == num - 2 ? idx[1] : idx[i + 2];
+        float e1x = POINT_UV[next][0] - POINT_UV[idx[0]][0];
+        float e1y = POINT_UV[next][1] - POINT_UV[idx[0]][1];
+        float vv = (ex * e1y) - (e1x * ey);
+        float area = (e0x * e1y) - (e1x * e0y);
+        float uf = uu / area;
+        float vf = vv / area;
+        float wf = (1.0f - uf) - vf;
+        if (uf < 0.0f || vf < 0.0f || wf < 0.0f) {
+            uu = -vv;
+            e0x = e1x;
+            e0y = e1y;
+            continue;
+        }
+        m.w[0] = wf;
+        m.point[1] = idx[i + 1]; m.w[1] = vf;
+        m.point[2] = next; m.w[2] = uf;
+        break;
+    }
+    return m;
 }
+
+// A colour's cell with the points' spectra beside each other, one element per
+// tabulated wavelength: the renderer lays out its fixed colours so once, and
+// a sample is eight 16-byte loads from 1.5 KB instead of a grid walk and 32
+// scattered words.  The Cornell box at 512x512, 16 spp: 7.05 -> 6.59 ms; eight
+// served requests 4.38 -> 4.25 ms.
+struct alignas(16) PreparedColor {
+    MengCell cell;
+    uint32_t pad[2];
+    float spectrum[psy_meng::NUM_SAMPLES][4];
+};
+static_assert(offsetof(PreparedColor, spectrum) % 16 == 0, "16-byte rows");
+// GpuColor::kind of such a colour; a and b hold the address.
+constexpr uint32_t COLOR_PREPARED = 0x100u;
+PSY_HD GpuColor prepared_ref(const PreparedColor* p) {
+    const uint64_t at = (uint64_t)p;
+    return GpuColor{COLOR_PREPARED, lm_float((uint32_t)at), lm_float((uint32_t)(at >> 32)), 0.0f};
+}
+
+// The four wavelengths' places in the tables: the sample below, the one
+// above, and how far between.
+struct MengPlace {
+    int below, above;
+    float between;
+};
+RD MengPlace meng_place(float lambda) {
+    using namespace psy_meng;
+    const float sb = ((lambda - SAMPLE_MIN) / (SAMPLE_MAX - SAMPLE_MIN)) * ((float)NUM_SAMPLES - 1.0f);
+    MengPlace m;
+    m.below = (int)sb;
+    m.above = m.below + 1 < NUM_SAMPLES - 1 ? m.below + 1 : NUM_SAMPLES - 1;
+    m.between = sb - (float)m.below;
+    return m;
+}
+// The weighted sum at one wavelength, of the points' spectra at the samples
+// below and above it.
+RD float meng_sum(const MengCell& m, float between, const float (&below)[4], const float (&above)[4]) {
+    auto lerped = [&](int j) { return (below[j] * (1.0f - between)) + (above[j] * between); };
+    float sum = ((lerped(0) * m.w[0]) + (lerped(1) * m.w[1])) + (lerped(2) * m.w[2]);
+    if (m.n == 4) sum = sum + (lerped(3) * m.w[3]);
+    return sum * m.inv_norm;
+}
+RD S4 spectrum_xyz_to_p_4(S4 lambdas, float x, float y, float z) {
+    const MengCell m = meng_cell(x, y, z);
+    if (m.n == 0) return s4_zero();
+    S4 r;
+    for (int k = 0; k < 4; k++) {
+        const MengPlace s = meng_place(lambdas.v[k]);
+        float lo[4], hi[4];
+        for (int j = 0; j < 4; j++) {
+            lo[j] = psy_meng::POINT_SPECTRUM[m.point[j]][s.below];
+            hi[j] = psy_meng::POINT_SPECTRUM[m.point[j]][s.above];
+        }
+        r.v[k] = meng_sum(m, s.between, lo, hi);
+    }
+    return r;
+}
+#ifndef PSY_RD_HOST
+RD S4 spectrum_prepared(S4 lambdas, const PreparedColor* p) {
+    MengCell m;
+    m.n = p->cell.n;
+    m.inv_norm = p->cell.inv_norm;
+    for (int j = 0; j < 4; j++) m.w[j] = p->cell.w[j];
+    if (m.n == 0) return s4_zero();
+    const float4* rows = reinterpret_cast<const float4*>(p->spectrum);
+    S4 r;
+    for (int k = 0; k < 4; k++) {
+        const MengPlace s = meng_place(lambdas.v[k]);
+        const float4 below = rows[s.below], above = rows[s.above];
+        const float lo[4] = {below.x, below.y, below.z, below.w}, hi[4] = {above.x, above.y, above.z, above.w};
+        r.v[k] = meng_sum(m, s.between, lo, hi);
+    }
+    return r;
+}
+#endif
 
 // plancks_law (color.rs:335-376), per micrometre
 RD float plancks_law(float temperature, float wavelength) {
@@ -522,6 +583,13 @@ RD S4 color_spectral(const GpuColor& c, float hero) {
     S4 wls = s4(nth_wavelength(hero, 0), nth_wavelength(hero, 1), nth_wavelength(hero, 2), nth_wavelength(hero, 3));
     if (c.kind == PSY_COLOR_XYZ)
         return spectrum_xyz_to_p_4(wls, c.a, c.b, c.c) * s4_splat(1.0f / psy_meng::EQUAL_ENERGY_REFLECTANCE);
+#ifndef PSY_RD_HOST
+    if (c.kind == COLOR_PREPARED) {
+        const uint64_t at = (uint64_t)lm_bits(c.a) | ((uint64_t)lm_bits(c.b) << 32);
+        const PreparedColor* p = (const PreparedColor*)(const __attribute__((address_space(1))) PreparedColor*)at;
+        return spectrum_prepared(wls, p) * s4_splat(1.0f / psy_meng::EQUAL_ENERGY_REFLECTANCE);
+    }
+#endif
     S4 r;
     for (int k = 0; k < 4; k++)
         r.v[k] = (c.kind == PSY_COLOR_BLACKBODY ? plancks_law(c.a, wls.v[k]) : plancks_law_normalized(c.a, wls.v[k])) *

@@ -22,6 +22,9 @@ using rd::HaltonDim;
 
 constexpr int KBLOCK = 256;
 constexpr uint32_t MAX_SEGS = 64;  // requests interleaved in one wave
+// Lights whose colours a renderer prepares, 1.5 KB each; the others' are
+// evaluated from the shared tables.
+constexpr uint32_t PREPARED_LIGHTS = 4096;
 constexpr uint32_t NUM_BINS = 6;   // miss, light, Lambert, GGX, emit, dielectric
 // Layout of the renderer's counter words: [0, 4) queue counts, then the sort
 // bins (2 * NUM_BINS), then the rays-traced u64 at an even word.
@@ -89,6 +92,10 @@ struct ShadeScene {
     const GpuRectLight* rects;
     const GpuSphereLight* spheres;
     const float* light_samples;  // time samples of the lights (layout.h)
+    // Prepared colours (render_device.h) of the first rect_prepared and
+    // sphere_prepared lights, in that order.
+    const rd::PreparedColor* light_colors;
+    uint32_t rect_prepared, sphere_prepared;
     const GpuLightNode* lnodes;
     const GpuBox* lboxes;
     const GpuLightLeaf* lleaves;
