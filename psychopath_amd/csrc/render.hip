@@ -232,51 +232,77 @@ __device__ __forceinline__ uint32_t hit_key(const ShadeScene& sc, const Hits& h,
     return 2u + (inst.shader == PSY_NONE ? sc.unassigned.kind : sc.shaders[inst.shader].kind);
 }
 
-// Counting sort of the closest hits by key, in two kernels over the same
-// block partition: block b takes queue entries [b*chunk, (b+1)*chunk).
-// sort_count adds each block's per-key counts to bins[0, NUM_BINS);
-// sort_scatter reserves each block's range in every bin with one atomic on
-// bins[NUM_BINS, 2 * NUM_BINS) and places the block's entries with LDS
-// counters.
-__device__ __forceinline__ uint32_t sort_chunk(uint32_t n) {
-    return (n + gridDim.x - 1) / gridDim.x;
-}
-
-__global__ __launch_bounds__(KBLOCK) void sort_count_kernel(ShadeScene sc, Hits h, const uint32_t* count,
-                                                            uint32_t* bins) {
-    __shared__ uint32_t local[NUM_BINS];
-    if (threadIdx.x < NUM_BINS) local[threadIdx.x] = 0u;
-    __syncthreads();
-    const uint32_t n = *count;
-    const uint32_t chunk = sort_chunk(n);
-    const uint32_t q0 = blockIdx.x * chunk, q1 = min(n, q0 + chunk);
-    for (uint32_t q = q0 + threadIdx.x; q < q1; q += blockDim.x) atomicAdd(&local[hit_key(sc, h, q)], 1u);
-    __syncthreads();
-    if (threadIdx.x < NUM_BINS && local[threadIdx.x] != 0u) atomicAdd(&bins[threadIdx.x], local[threadIdx.x]);
-}
-
-__global__ __launch_bounds__(KBLOCK) void sort_scatter_kernel(ShadeScene sc, Hits h, const uint32_t* count,
-                                                              uint32_t* bins, uint32_t* order) {
+// Closest hits by key: every key has a region of `capacity` entries in
+// `order`, and bins[key] counts it, so one pass both counts and places.  A
+// block takes tiles of 4 entries a lane (16 in long queues, where a tile per
+// atomic counts) and keeps their keys while it reserves the tile's part of
+// every region.  Counting and scattering in two kernels over 1,024 blocks
+// whatever the queue took 0.33 ms of the Cornell box at 512x512, 16 spp and
+// 0.15 ms at 64x64, 4 spp, where the blocks' atomics on three counters waited
+// for one another; this takes 0.19 and 0.046 ms.
+constexpr uint32_t SORT_LONG = 1u << 20;
+__global__ __launch_bounds__(KBLOCK) void sort_kernel(ShadeScene sc, Hits h, const uint32_t* count, uint32_t* bins,
+                                                      uint32_t* order, uint32_t capacity) {
+    static_assert(NUM_BINS <= 15, "four bits a key, 15: no entry");
     __shared__ uint32_t local[NUM_BINS], base[NUM_BINS];
-    if (threadIdx.x < NUM_BINS) local[threadIdx.x] = 0u;
-    __syncthreads();
     const uint32_t n = *count;
-    const uint32_t chunk = sort_chunk(n);
-    const uint32_t q0 = blockIdx.x * chunk, q1 = min(n, q0 + chunk);
-    for (uint32_t q = q0 + threadIdx.x; q < q1; q += blockDim.x) atomicAdd(&local[hit_key(sc, h, q)], 1u);
-    __syncthreads();
-    if (threadIdx.x < NUM_BINS) {
-        uint32_t start = 0;
-        for (uint32_t b = 0; b < threadIdx.x; b++) start += bins[b];
-        base[threadIdx.x] = local[threadIdx.x] ? start + atomicAdd(&bins[NUM_BINS + threadIdx.x], local[threadIdx.x])
-                                               : 0u;
-        local[threadIdx.x] = 0u;
+    const uint32_t per = n >= SORT_LONG ? 16u : 4u;  // entries per lane
+    const uint32_t tile = per * (uint32_t)KBLOCK;
+    for (uint64_t t0 = (uint64_t)blockIdx.x * tile; t0 < n; t0 += (uint64_t)gridDim.x * tile) {
+        if (threadIdx.x < NUM_BINS) local[threadIdx.x] = 0u;
+        __syncthreads();
+        const uint32_t q0 = (uint32_t)t0 + threadIdx.x;
+        uint64_t keys = ~0ull;
+        for (uint32_t j = 0; j < per; j += 4) {
+#pragma unroll
+            for (uint32_t i = 0; i < 4; i++) {
+                const uint32_t q = q0 + (j + i) * (uint32_t)KBLOCK;
+                if (q >= n) continue;
+                const uint32_t key = hit_key(sc, h, q);
+                keys ^= (uint64_t)(key ^ 15u) << (4u * (j + i));
+                atomicAdd(&local[key], 1u);
+            }
+        }
+        __syncthreads();
+        if (threadIdx.x < NUM_BINS) {
+            base[threadIdx.x] = local[threadIdx.x] ? atomicAdd(&bins[threadIdx.x], local[threadIdx.x]) : 0u;
+            local[threadIdx.x] = 0u;
+        }
+        __syncthreads();
+        for (uint32_t j = 0; j < per; j++) {
+            const uint32_t key = (uint32_t)(keys >> (4u * j)) & 15u;
+            if (key == 15u) continue;
+            order[(uint64_t)key * capacity + base[key] + atomicAdd(&local[key], 1u)] = q0 + j * (uint32_t)KBLOCK;
+        }
+        __syncthreads();
     }
-    __syncthreads();
-    for (uint32_t q = q0 + threadIdx.x; q < q1; q += blockDim.x) {
-        const uint32_t key = hit_key(sc, h, q);
-        order[base[key] + atomicAdd(&local[key], 1u)] = q;
+}
+// Where each key's entries end when its regions are taken one after another
+// (uniform: read once, into scalar registers).
+struct SortedRuns {
+    uint32_t end[NUM_BINS];
+};
+__device__ __forceinline__ SortedRuns sorted_runs(const uint32_t* bins) {
+    SortedRuns r;
+    uint32_t sum = 0;
+#pragma unroll
+    for (uint32_t k = 0; k < NUM_BINS; k++) {
+        sum += (uint32_t)__builtin_amdgcn_readfirstlane((int)bins[k]);
+        r.end[k] = sum;
     }
+    return r;
+}
+// Entry i of that sequence.
+__device__ __forceinline__ uint32_t sorted_entry(const SortedRuns& r, const uint32_t* order, uint32_t capacity,
+                                                 uint32_t i) {
+    uint32_t key = 0, start = 0;
+#pragma unroll
+    for (uint32_t k = 0; k + 1 < NUM_BINS; k++)
+        if (i >= r.end[k]) {
+            key = k + 1;
+            start = r.end[k];
+        }
+    return order[(uint64_t)key * capacity + (i - start)];
 }
 
 // Surface intersection data (SurfaceIntersectionData, src/surface/mod.rs:
@@ -737,9 +763,10 @@ __device__ __forceinline__ void shade_path(const ShadeScene& sc, const ReqParams
 // the same thing.
 template <int MINW>
 __global__ __launch_bounds__(KBLOCK) __attribute__((amdgpu_waves_per_eu(MINW))) void shade_kernel(
-    ShadeScene sc, const ReqParams* reqs, Paths P, Queue qa, Hits h, const uint32_t* order, Queue qa_out,
-    Queue qs_out) {
+    ShadeScene sc, const ReqParams* reqs, Paths P, Queue qa, Hits h, const uint32_t* order, const uint32_t* bins,
+    uint32_t capacity, Queue qa_out, Queue qs_out) {
     const uint32_t n = *qa.count;
+    const SortedRuns runs = sorted_runs(bins);
     const uint32_t stride = gridDim.x * blockDim.x;
     // Every thread of a block runs the loop the same number of times, so the
     // block-wide appends see all of them.  One atomic per block and queue:
@@ -755,7 +782,7 @@ __global__ __launch_bounds__(KBLOCK) __attribute__((amdgpu_waves_per_eu(MINW))) 
         float ptime = 0.0f;
         uint32_t p = 0;
         if (i < n) {
-            const uint32_t q = order ? order[i] : i;
+            const uint32_t q = order ? sorted_entry(runs, order, capacity, i) : i;
             p = qa.path[q];
             const ReqParams rp = reqs[P.req[p]];
             PathRegs ps;
@@ -1170,7 +1197,7 @@ int enqueue_wave(psy_renderer* r, uint32_t steps) {
             a.clear0 = qa_out.count;
             a.clear1 = qs_out.count;
             a.clear_run = r->counts + COUNTS_BINS;
-            a.clear_run_n = 2 * NUM_BINS;
+            a.clear_run_n = NUM_BINS;
             return a;
         };
         if (!tally) {
@@ -1195,12 +1222,8 @@ int enqueue_wave(psy_renderer* r, uint32_t steps) {
         const uint32_t* order = nullptr;
         if (r->sort_materials) {
             rc = staged(r, ST_SORT, [&]() -> int {
-                const uint32_t sgrid = std::min<uint32_t>(grid, 1024);
-                hipLaunchKernelGGL(sort_count_kernel, dim3(sgrid), dim3(KBLOCK), 0, s, r->sc, r->ha, qa_in.count,
-                                   r->counts + COUNTS_BINS);
-                PSY_HIP(hipGetLastError());
-                hipLaunchKernelGGL(sort_scatter_kernel, dim3(sgrid), dim3(KBLOCK), 0, s, r->sc, r->ha, qa_in.count,
-                                   r->counts + COUNTS_BINS, r->order);
+                hipLaunchKernelGGL(sort_kernel, dim3(std::min<uint32_t>(grid, 1024)), dim3(KBLOCK), 0, s, r->sc, r->ha,
+                                   qa_in.count, r->counts + COUNTS_BINS, r->order, (uint32_t)r->capacity);
                 PSY_HIP(hipGetLastError());
                 return PSY_OK;
             });
@@ -1212,8 +1235,8 @@ int enqueue_wave(psy_renderer* r, uint32_t steps) {
                      : r->shade_waves == 2 ? shade_kernel<2>
                                            : shade_kernel<1>;
         rc = staged(r, ST_SHADE, [&]() -> int {
-            hipLaunchKernelGGL(shade, dim3(grid), dim3(KBLOCK), 0, s, r->sc, r->reqs, r->P, qa_in, r->ha, order, qa_out,
-                               qs_out);
+            hipLaunchKernelGGL(shade, dim3(grid), dim3(KBLOCK), 0, s, r->sc, r->reqs, r->P, qa_in, r->ha, order,
+                               r->counts + COUNTS_BINS, (uint32_t)r->capacity, qa_out, qs_out);
             PSY_HIP(hipGetLastError());
             return PSY_OK;
         });
@@ -1483,7 +1506,12 @@ int psy_renderer_create(const psy_scene* scene_c, const psy_world_desc* world, u
     for (int k = 0; k < 4 && !rc; k++) rc = r->alloc(hf[k], C);
     if (!rc) rc = r->alloc(&r->ha.prim, C);
     if (!rc) rc = r->alloc(&r->ha.inst, C);
-    if (!rc) rc = r->alloc(&r->order, C);
+    // (regions up to the last key that the scene's surfaces can have)
+    uint32_t keys = 2;
+    for (const GpuInstance& gi : scene->host.instances)
+        if (gi.kind == PSY_OBJECT_MESH)
+            keys = std::max(keys, 3u + (gi.shader == PSY_NONE ? (uint32_t)PSY_SHADER_EMIT : shaders[gi.shader].kind));
+    if (!rc) rc = r->alloc(&r->order, (uint64_t)keys * C);
     if (!rc) rc = r->alloc(&r->counts, COUNTS_WORDS);
     if (!rc) rc = r->alloc(&r->wave_idx, 1);
     if (!rc) rc = r->alloc(&r->work, 2 * TRACE_WORK_WORDS);
