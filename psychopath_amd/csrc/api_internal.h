@@ -25,8 +25,8 @@ int fail(int code, const std::string& msg);
     } while (0)
 
 // The launch shape of a new tracer or renderer: as many waves as the kernel's
-// build allows on a CU (24 is more than any 4-wave build does, 20 on static
-// scenes and 16 with transforms), and descent rounds that end when half of a
+// build allows on a CU (24 is more than the 16 to 20 of the 4-wave builds),
+// and descent rounds that end when half of a
 // wave waits.  Against 16 waves and descents to the last lane: 16.7M
 // incoherent rays on the 1M-triangle sphere 5.15 -> 3.37 ms, 4.0M shadow rays
 // 1.28 -> 0.93 ms, 1M rays on the motion scene 1.63 -> 1.36 ms and its
