@@ -69,7 +69,7 @@ TraceArgs scene_args(const psy_scene* s) {
     a.groups = s->host.nested ? s->groups : nullptr;
     a.top_root = s->host.top_root;
     a.node_count = (uint32_t)s->host.nodes.size();
-    a.nan_boxes = s->host.nan_boxes ? 1u : 0u;
+    a.odd_boxes = s->host.odd_boxes ? 1u : 0u;
     return a;
 }
 

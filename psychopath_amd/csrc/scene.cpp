@@ -105,25 +105,34 @@ const NodeSlots& node_slots() {
 }
 
 // One sample's four boxes with their children moved to their slots.  Returns
-// whether a plane is NaN.
-bool slot_boxes(const float* in, const uint8_t* child, float* out) {
+// whether a child's box is one that slab_finite does not serve: it needs
+// low <= high on every axis, which a NaN plane fails and so does the empty
+// box [+inf, -inf] that an instance has whose transform cannot be inverted or
+// whose object's bounds turn to NaN under it (slab, which orders the planes
+// itself, hits that one).  Planes that are lerped (`sampled`) must be finite
+// as well: an infinite one times a weight of zero is NaN.
+bool slot_boxes(const float* in, const uint8_t* child, bool sampled, float* out) {
     const float inf = __builtin_huge_valf();
-    bool nan = false;
-    for (int k = 0; k < 24; k++) nan |= in[k] != in[k];
     if (child[1] == 1) {  // the left side has two children: slots as children
         std::memcpy(out, in, 24 * sizeof(float));
         if (child[3] == 4)
             for (int p = 0; p < 6; p++) out[4 * p + 3] = inf;
-        return nan;
+    } else {
+        const bool two = child[3] == 4;
+        for (int p = 0; p < 6; p++) {
+            out[4 * p] = in[4 * p];
+            out[4 * p + 1] = inf;
+            out[4 * p + 2] = in[4 * p + 1];
+            out[4 * p + 3] = two ? inf : in[4 * p + 2];
+        }
     }
-    const bool two = child[3] == 4;
-    for (int p = 0; p < 6; p++) {
-        out[4 * p] = in[4 * p];
-        out[4 * p + 1] = inf;
-        out[4 * p + 2] = in[4 * p + 1];
-        out[4 * p + 3] = two ? inf : in[4 * p + 2];
-    }
-    return nan;
+    bool odd = false;
+    for (int p = 0; p < 6; p += 2)
+        for (int k = 0; k < 4; k++) odd |= !(out[4 * p + k] <= out[4 * p + 4 + k]);
+    if (sampled)
+        for (int p = 0; p < 6; p++)
+            for (int k = 0; k < 4; k++) odd |= child[k] != 4 && !(std::fabs(out[4 * p + k]) < inf);
+    return odd;
 }
 
 // Appends `bvh` to the scene arrays in the device form (layout.h: children
@@ -138,7 +147,7 @@ uint32_t append_bvh(PackedScene& s, const HostBvh4& bvh) {
     for (const GpuNode& n : bvh.nodes) {
         const uint32_t code = (n.meta >> 16) & 0x3fu, blen = (n.meta >> 8) & 0xffu;
         const uint8_t* child = t.child[code];
-        if (slot_boxes(n.lo_x, child, out->lo_x)) s.nan_boxes = true;
+        if (slot_boxes(n.lo_x, child, false, out->lo_x)) s.odd_boxes = true;
         for (int k = 0; k < 4; k++) {
             uint32_t ref = REF_ABSENT;
             if (child[k] < 4) {
@@ -152,7 +161,7 @@ uint32_t append_bvh(PackedScene& s, const HostBvh4& bvh) {
         if (n.motion != REF_EMPTY) {
             out->motion += motion_base;
             for (uint32_t k = 0; k < blen; k++)
-                if (slot_boxes(bvh.motion[n.motion + k].lo_x, child, s.motion[out->motion + k].lo_x)) s.nan_boxes = true;
+                if (slot_boxes(bvh.motion[n.motion + k].lo_x, child, true, s.motion[out->motion + k].lo_x)) s.odd_boxes = true;
         }
         out++;
     }

@@ -45,7 +45,7 @@ struct PackedScene {
     bool has_motion = false;    // time-sampled node bounds or vertices
     bool has_lights = false;    // some instance places a light
     bool has_normals = false;   // some mesh has shading normals
-    bool nan_boxes = false;     // some node bound is NaN
+    bool odd_boxes = false;     // some node's box is not one that slab_finite serves (scene.cpp)
     bool nested = false;        // sub-assemblies are traversed as nested BVHs (`groups`)
     uint32_t max_stack = 0;     // deepest pending-node count traversal can need
     uint32_t max_depth = 0;

@@ -38,7 +38,7 @@ struct TraceArgs {
     const GpuGroup* groups;      // nested scenes: instance paths (layout.h), else NULL
     uint32_t top_root;
     uint32_t node_count;
-    uint32_t nan_boxes;          // some node bound is NaN
+    uint32_t odd_boxes;          // some node's box needs the full test (PackedScene)
     // rays (device)
     const float *ox, *oy, *oz, *dx, *dy, *dz, *time, *max_t;
     const uint8_t* flags;

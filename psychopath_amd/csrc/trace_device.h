@@ -28,9 +28,9 @@ __device__ __forceinline__ bool slab(float lox, float hix, float loy, float hiy,
 }
 
 // The same test for a ray whose origin, inverse direction and far end hold no
-// NaN and no infinity but a far end of +inf, against planes without NaN, the
-// planes given as the ray meets them (near: the low plane where the
-// direction is positive).  Without NaN the minima and maxima need no operand
+// NaN and no infinity but a far end of +inf, against boxes whose low planes
+// are not above their high ones (so without NaN), the planes given as the ray
+// meets them (near: the low plane where the direction is positive).  Without NaN the minima and maxima need no operand
 // order, and of a box's two planes on an axis the near one's distance is
 // never the larger (rounding is monotonic), so this returns what slab does in
 // 17 instructions instead of 35.

@@ -183,7 +183,7 @@ void trace_persistent_kernel(TraceArgs a, unsigned int* work, uint32_t refill_mi
         near_y = di.y < 0.0f ? 16u : 0u;
         near_z = di.z < 0.0f ? 16u : 0u;
         down = octant_of(di) << REF_AXIS_SHIFT;
-        finite = !a.nan_boxes && !(tmax != tmax) && finite_ray(lo, di);
+        finite = !a.odd_boxes && !(tmax != tmax) && finite_ray(lo, di);
     };
     uint32_t cur = REF_EMPTY;
     bool in_inst = false;

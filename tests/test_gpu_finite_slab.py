@@ -2,7 +2,9 @@
 test of finite rays does not serve (zero direction components, origins in a
 box's planes, infinities, NaN) and, in the same waves, rays that it does,
 must give the records of the one-lane grid kernel, which has the reference's
-box test only; on the static scene without NaN also the oracle's."""
+box test only; on the static scene without NaN also the oracle's.  Scenes
+whose boxes the reduced test does not serve (NaN, empty, or infinite where
+they are lerped) must take the full one."""
 
 import numpy as np
 import pytest
@@ -99,3 +101,82 @@ def test_box_tests_agree(kind):
         s = (w["kind"] == 2) & np.isfinite(w["t"])  # (a NaN hit of a NaN ray: which of many is not defined)
         for k in ("t", "b0", "b1", "b2", "prim_id"):
             assert np.array_equal(want[k][s], w[k][s]), k
+
+
+def odd_scene(kind):
+    """A plain instance beside one whose box in the instance BVH, or in a
+    time-sampled node, is empty ([+inf, -inf]) or infinite."""
+    v, f = steps_mesh()
+    place = np.array([[1, 0, 0, -3, 0, 1, 0, 0, 0, 0, 1, -6]], np.float32)
+    flat = np.array([[1, 0, 0, 0, 0, 1, 0, 0, 0, 0, 0, 0]], np.float32)
+    meshes, instances = [(v, f)], [(0, None)]
+    if kind == "flattened":
+        instances.append((0, flat))
+    elif kind == "flattened, moving":
+        instances.append((0, np.concatenate([flat, flat + np.eye(1, 12, 3, dtype=np.float32)])))
+    elif kind == "scaled to nothing":
+        instances.append((0, np.zeros((1, 12), np.float32)))
+    elif kind == "one leaf with a NaN vertex":
+        w = np.array([(2, 2, 6), (9, 2, 6), (2, 9, 6), (3, 3, 7), (8, 3, 7), (np.nan,) * 3], np.float32)
+        meshes.append((w, np.array([(0, 1, 2), (3, 4, 5)], np.uint32)))
+        instances.append((1, place))
+    elif kind == "all NaN":
+        meshes.append((np.full((3, 3), np.nan, np.float32), np.array([(0, 1, 2)], np.uint32)))
+        instances.append((1, place))
+    elif kind == "both infinities":
+        w = v.copy()
+        w[5], w[90] = np.inf, -np.inf
+        meshes.append((w, f))
+        instances.append((1, place))
+    else:  # infinite planes in time samples
+        w = np.stack([v, v + 1])
+        w[0, 5], w[1, 90], w[:, 200] = np.inf, -np.inf, np.inf
+        meshes.append((w, f))
+        instances.append((1, None))
+    return meshes, instances
+
+
+@pytest.mark.parametrize("kind", ["flattened", "flattened, moving", "scaled to nothing", "one leaf with a NaN vertex",
+                                  "all NaN", "both infinities", "infinite, moving"])
+def test_odd_boxes_take_the_full_test(kind):
+    from oracle.psyref import OracleScene
+    meshes, instances = odd_scene(kind)
+    a, o = Assembly(), OracleScene()
+    for m in meshes:
+        a.add_mesh(Mesh(*m))
+        o.add_mesh(*m)
+    for mesh, xf in instances:
+        a.add_instance(mesh, xf)
+        o.add_instance(mesh, xf)
+    o.build()
+    tracer = Tracer(a.build(), max_batch=1 << 14)
+    # All kinds of rays, then finite ones only, in whole waves of their own:
+    # no lane of these forces the full test on the others.
+    batch = rays()
+    rng = np.random.default_rng(6)
+    n = 4096
+    p, q = (rng.uniform(-1, 13, (n, 3)).astype(np.float32) for _ in range(2))
+    t = (np.arange(n) % 3 / 2).astype(np.float32)
+    fields = [np.concatenate(x) for x in zip((getattr(batch, k) for k in ("ox", "oy", "oz", "dx", "dy", "dz", "time",
+                                                                           "max_t")),
+                                             (*p.T, *(q - p).T, t, np.full(n, np.inf, np.float32)))]
+    batch = RayBatch(*fields, np.concatenate([batch.flags, np.zeros(n, np.uint8)]))
+    dr = DeviceRays(batch)
+    want = records(tracer, (1, 1, 1, 8, 4, 0), dr)
+    w = o.trace({k: getattr(batch, k) for k in ("ox", "oy", "oz", "dx", "dy", "dz", "time", "max_t")}
+                | {"occlusion": batch.flags})
+    finite = slice(len(batch) - n, None)
+    assert np.array_equal(want["kind"][finite], w["kind"][finite])
+    # (which hit a ray ends on that met a NaN one is not defined)
+    s = (w["kind"] == 2) & np.isfinite(w["t"]) & np.isfinite(want["t"])
+    s[:finite.start] = False
+    for k in ("t", "prim_id", "inst_id"):
+        assert np.array_equal(want[k][s], w[k][s]), k
+    alone = DeviceRays(batch.slice(finite.start, len(batch)))
+    tracer.set_tuning(1, 1, 1, 8, 4, 0)
+    visits = tracer.trace_counted(alone, DeviceHitRecords(n))
+    assert visits["instance_visits"] > n
+    for shape in SHAPES:
+        assert records(tracer, shape, dr).tobytes() == want.tobytes(), (kind, shape)
+        assert records(tracer, shape, alone).tobytes() == want[finite].tobytes(), (kind, shape)
+        assert tracer.trace_counted(alone, DeviceHitRecords(n)) == visits, (kind, shape)
