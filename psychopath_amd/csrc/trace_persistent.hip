@@ -121,8 +121,9 @@ __device__ __forceinline__ void level_local_ray(const TraceArgs& a, const GpuGro
 }
 
 // RING: LDS stack entries per lane, a power of two.  BIG: the node array is
-// longer than 4 GB, so node addresses take 64-bit offsets.
-template <bool COUNT, bool XF, bool MOTION, uint32_t RING, int MIN_WAVES, bool COOP, bool NESTED, bool BIG>
+// longer than 4 GB, so node addresses take 64-bit offsets.  DIRECT: the scene
+// is one mesh instance without a transform (its instance BVH is that leaf).
+template <bool COUNT, bool XF, bool MOTION, uint32_t RING, int MIN_WAVES, bool COOP, bool NESTED, bool BIG, bool DIRECT>
 __global__ __launch_bounds__(WAVE) __attribute__((amdgpu_waves_per_eu(MIN_WAVES)))
 void trace_persistent_kernel(TraceArgs a, unsigned int* work, uint32_t refill_min, uint32_t leaf_min) {
     __shared__ uint32_t lds_stack[RING * WAVE];
@@ -150,16 +151,17 @@ void trace_persistent_kernel(TraceArgs a, unsigned int* work, uint32_t refill_mi
             if (a.tally) atomicAdd(a.tally, (unsigned long long)n);
         }
     }
-    // A scene that is one mesh instance without a transform (its instance BVH
-    // is that leaf) needs no walk to it: its rays start on the mesh's root.
-    // That saves every ray a leaf round with two dependent loads: 16.7M
-    // incoherent rays on the 1M-triangle sphere 3.39 -> 3.24 ms, 4.0M shadow
-    // rays 0.943 -> 0.895 ms.  (The build takes 100 registers and 16 waves per
-    // CU; held to 96 and 20 waves it is back at 3.39 and 0.94.)
-    const bool direct = !XF && !NESTED && a.top_root != REF_EMPTY && (a.top_root & REF_LEAF) != 0u;
+    // A scene that is one untransformed instance needs no walk to it: its rays
+    // start on the mesh's root.  That saves every ray a leaf round with two
+    // dependent loads and is worth the four registers (100 instead of 96, so
+    // 16 waves per CU instead of 20): 16.7M incoherent rays on the
+    // 1M-triangle sphere 3.39 -> 3.24 ms, 4.0M shadow rays 0.943 -> 0.895.  A
+    // build of its own, so that other static scenes keep their waves: 4.2M
+    // rays on the sphere cut into 16 meshes take 1.51 ms, and took 1.64 where
+    // one build chose at run time.
     GpuInstance only{};
     GpuMesh only_mesh{};
-    if (direct) {
+    if (DIRECT) {
         only = a.instances[(a.top_root & ~REF_LEAF) >> 2];
         only_mesh = a.meshes[only.mesh];
     }
@@ -275,7 +277,7 @@ void trace_persistent_kernel(TraceArgs a, unsigned int* work, uint32_t refill_mi
                     sp = 0;
                     bot = 0;
                     in_inst = false;
-                    if (direct) {
+                    if (DIRECT) {
                         if (COUNT) c_inst++;
                         cur = only_mesh.root;
                         in_inst = true;
@@ -688,32 +690,32 @@ hipError_t launch_resident(const TraceArgs& a, unsigned int* work, const TraceTu
     return hipGetLastError();
 }
 
-template <bool COUNT, bool XF, bool MOTION, uint32_t RING, bool NESTED, bool BIG>
+template <bool COUNT, bool XF, bool MOTION, uint32_t RING, bool NESTED, bool BIG, bool DIRECT>
 hipError_t launch_one(const TraceArgs& a, unsigned int* work, const TraceTuning& tune, hipStream_t s) {
     // Register budget: 8 waves per SIMD caps the kernel at 64 VGPRs (the
     // compiler keeps the rest in private memory), 4 lets it use up to 128.
     // The cooperative node fetch serves static single-level scenes.
     if constexpr (!COUNT && !MOTION && !NESTED) {
         if (tune.coop) {
-            if (tune.occupancy >= 8) return launch_resident<&trace_persistent_kernel<false, XF, false, RING, 8, true, false, false>>(a, work, tune, s);
-            return launch_resident<&trace_persistent_kernel<false, XF, false, RING, 4, true, false, false>>(a, work, tune, s);
+            if (tune.occupancy >= 8) return launch_resident<&trace_persistent_kernel<false, XF, false, RING, 8, true, false, false, DIRECT>>(a, work, tune, s);
+            return launch_resident<&trace_persistent_kernel<false, XF, false, RING, 4, true, false, false, DIRECT>>(a, work, tune, s);
         }
     }
     if constexpr (!COUNT && !BIG) {
-        if (tune.occupancy >= 8) return launch_resident<&trace_persistent_kernel<false, XF, MOTION, RING, 8, false, NESTED, false>>(a, work, tune, s);
+        if (tune.occupancy >= 8) return launch_resident<&trace_persistent_kernel<false, XF, MOTION, RING, 8, false, NESTED, false, DIRECT>>(a, work, tune, s);
     }
-    return launch_resident<&trace_persistent_kernel<COUNT, XF, MOTION, RING, 4, false, NESTED, BIG>>(a, work, tune, s);
+    return launch_resident<&trace_persistent_kernel<COUNT, XF, MOTION, RING, 4, false, NESTED, BIG, DIRECT>>(a, work, tune, s);
 }
 
-template <bool COUNT, bool XF, bool MOTION, bool NESTED>
+template <bool COUNT, bool XF, bool MOTION, bool NESTED, bool DIRECT>
 hipError_t launch_depth(const TraceArgs& a, unsigned int* work, const TraceTuning& tune, hipStream_t s) {
     if constexpr (COUNT || NESTED) {
-        return launch_one<COUNT, XF, MOTION, 16, NESTED, false>(a, work, tune, s);
+        return launch_one<COUNT, XF, MOTION, 16, NESTED, false, DIRECT>(a, work, tune, s);
     } else {
         switch (tune.lds_depth) {
-            case 8: return launch_one<COUNT, XF, MOTION, 8, false, false>(a, work, tune, s);
-            case 24: return launch_one<COUNT, XF, MOTION, 32, false, false>(a, work, tune, s);
-            default: return launch_one<COUNT, XF, MOTION, 16, false, false>(a, work, tune, s);
+            case 8: return launch_one<COUNT, XF, MOTION, 8, false, false, DIRECT>(a, work, tune, s);
+            case 24: return launch_one<COUNT, XF, MOTION, 32, false, false, DIRECT>(a, work, tune, s);
+            default: return launch_one<COUNT, XF, MOTION, 16, false, false, DIRECT>(a, work, tune, s);
         }
     }
 }
@@ -724,18 +726,21 @@ hipError_t launch_feat(const TraceArgs& a, unsigned int* work, const TraceTuning
     // More than 4 GB of nodes: the most general build, with 64-bit node
     // offsets.
     if (a.node_count > (1u << 25)) {
-        if (a.groups) return launch_one<COUNT, true, true, 16, true, true>(a, work, tune, s);
-        return launch_one<COUNT, true, true, 16, false, true>(a, work, tune, s);
+        if (a.groups) return launch_one<COUNT, true, true, 16, true, true, false>(a, work, tune, s);
+        return launch_one<COUNT, true, true, 16, false, true, false>(a, work, tune, s);
     }
     // Nested scenes take the transform path, with or without time samples.
     if (a.groups) {
-        if (motion) return launch_depth<COUNT, true, true, true>(a, work, tune, s);
-        return launch_depth<COUNT, true, false, true>(a, work, tune, s);
+        if (motion) return launch_depth<COUNT, true, true, true, false>(a, work, tune, s);
+        return launch_depth<COUNT, true, false, true, false>(a, work, tune, s);
     }
-    if (xf && motion) return launch_depth<COUNT, true, true, false>(a, work, tune, s);
-    if (xf) return launch_depth<COUNT, true, false, false>(a, work, tune, s);
-    if (motion) return launch_depth<COUNT, false, true, false>(a, work, tune, s);
-    return launch_depth<COUNT, false, false, false>(a, work, tune, s);
+    if (xf && motion) return launch_depth<COUNT, true, true, false, false>(a, work, tune, s);
+    if (xf) return launch_depth<COUNT, true, false, false, false>(a, work, tune, s);
+    const bool direct = a.top_root != REF_EMPTY && (a.top_root & REF_LEAF);
+    if (motion && direct) return launch_depth<COUNT, false, true, false, true>(a, work, tune, s);
+    if (motion) return launch_depth<COUNT, false, true, false, false>(a, work, tune, s);
+    if (direct) return launch_depth<COUNT, false, false, false, true>(a, work, tune, s);
+    return launch_depth<COUNT, false, false, false, false>(a, work, tune, s);
 }
 
 }  // namespace
