@@ -253,9 +253,9 @@ typedef struct {
  * many as its registers and LDS let a unit hold), each starting
  * on its share of the rays and then taking chunks from a counter; lanes whose ray finished are
  * refilled from the wave's chunk once `refill_min` lanes of a wave are idle; `stack_lds` stack entries per lane
- * live in LDS (8, 16 or 24) and the rest in private memory; `simd_waves`
- * is the register budget, as resident waves per SIMD (4: up to 128 VGPRs,
- * 8: at most 64); `leaf_min` 0 lets each lane descend until it reaches a
+ * live in LDS (8, 16, or 24 for a ring of 32) and the rest in private memory;
+ * `simd_waves` is the register budget (4: up to 128 VGPRs, for four waves per
+ * SIMD at least; 8: the compiler's choice, for three to five); `leaf_min` 0 lets each lane descend until it reaches a
  * leaf or a node whose children all miss, 1..64 pops past such nodes inside
  * the descent and ends a wave's descent round once no lane stands on an
  * internal node or `leaf_min` lanes wait at a leaf.  The simple kernel runs

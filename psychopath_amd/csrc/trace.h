@@ -76,8 +76,8 @@ struct TraceTuning {
     uint32_t cus;          // compute units of the device
     uint32_t waves_per_cu; // wave64 workgroups launched per CU, at most as many as it holds
     uint32_t refill_min;  // idle lanes that trigger a refill (1..64)
-    uint32_t lds_depth;   // stack entries per lane kept in LDS (8, 16, 24)
-    uint32_t occupancy;   // register budget as waves per SIMD (4 or 8)
+    uint32_t lds_depth;   // stack entries per lane kept in LDS (8, 16, or 24 for 32)
+    uint32_t occupancy;   // register budget: 4 at most 128 VGPRs, 8 the compiler's choice
     uint32_t leaf_min;    // waiting lanes that end a descent round (1..64), 0: per-lane descents
     uint32_t coop;        // 1: wave-cooperative node fetch (static scenes)
 };

@@ -692,17 +692,22 @@ hipError_t launch_resident(const TraceArgs& a, unsigned int* work, const TraceTu
 
 template <bool COUNT, bool XF, bool MOTION, uint32_t RING, bool NESTED, bool BIG, bool DIRECT>
 hipError_t launch_one(const TraceArgs& a, unsigned int* work, const TraceTuning& tune, hipStream_t s) {
-    // Register budget: 8 waves per SIMD caps the kernel at 64 VGPRs (the
-    // compiler keeps the rest in private memory), 4 lets it use up to 128.
+    // Register budget: at most 128 VGPRs (four waves per SIMD), or what the
+    // compiler takes of its own (96 to 100 in static builds, 126 with
+    // transforms, up to 152 with time samples as well, which leaves three
+    // waves).  A budget of eight waves, 64 VGPRs, would spill in the node
+    // step: at 24 waves per CU and leaf_min 32, 4.2M rays on the 1M-triangle
+    // sphere took 1.98 ms so and 1.14 with 100 registers, 1M rays on the
+    // motion scene 2.62 and 0.88.
     // The cooperative node fetch serves static single-level scenes.
     if constexpr (!COUNT && !MOTION && !NESTED) {
         if (tune.coop) {
-            if (tune.occupancy >= 8) return launch_resident<&trace_persistent_kernel<false, XF, false, RING, 8, true, false, false, DIRECT>>(a, work, tune, s);
+            if (tune.occupancy >= 8) return launch_resident<&trace_persistent_kernel<false, XF, false, RING, 1, true, false, false, DIRECT>>(a, work, tune, s);
             return launch_resident<&trace_persistent_kernel<false, XF, false, RING, 4, true, false, false, DIRECT>>(a, work, tune, s);
         }
     }
     if constexpr (!COUNT && !BIG) {
-        if (tune.occupancy >= 8) return launch_resident<&trace_persistent_kernel<false, XF, MOTION, RING, 8, false, NESTED, false, DIRECT>>(a, work, tune, s);
+        if (tune.occupancy >= 8) return launch_resident<&trace_persistent_kernel<false, XF, MOTION, RING, 1, false, NESTED, false, DIRECT>>(a, work, tune, s);
     }
     return launch_resident<&trace_persistent_kernel<COUNT, XF, MOTION, RING, 4, false, NESTED, BIG, DIRECT>>(a, work, tune, s);
 }
