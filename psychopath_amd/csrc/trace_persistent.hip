@@ -665,7 +665,11 @@ __global__ void reset_work_kernel(unsigned int* work) { work[threadIdx.x * TRACE
 // wave that has to wait for another to end starts its share that late.
 // Launched at 24 per CU where 20 fit, 16.7M incoherent rays took 3.42 ms and
 // at 20 3.33; the motion scene's 1M rays 1.70 ms at 20 where 16 fit and 1.35
-// at 16.
+// at 16.  A CU hands out its LDS in LDS_GRANULE pieces, which the runtime's
+// answer leaves out: 18 waves with 8 KB fit, not 20 (4.2M rays on the
+// 1M-triangle sphere cut into 16 meshes, stack_lds 24: 1.50 ms at 18 waves,
+// 1.70 at 19 and 20).
+constexpr uint32_t LDS_PER_CU = 160u << 10, LDS_GRANULE = 1280;
 template <auto KERNEL>
 hipError_t launch_resident(const TraceArgs& a, unsigned int* work, const TraceTuning& tune, hipStream_t s) {
     static std::atomic<uint32_t> resident{0};
@@ -673,8 +677,11 @@ hipError_t launch_resident(const TraceArgs& a, unsigned int* work, const TraceTu
     if (per_cu == 0) {
         int blocks = 0;
         hipError_t e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&blocks, KERNEL, WAVE, 0);
+        hipFuncAttributes fa{};
+        if (e == hipSuccess) e = hipFuncGetAttributes(&fa, reinterpret_cast<const void*>(KERNEL));
         if (e != hipSuccess) return e;
-        per_cu = (uint32_t)std::max(1, blocks);
+        const uint32_t pieces = ((uint32_t)fa.sharedSizeBytes + LDS_GRANULE - 1u) / LDS_GRANULE;
+        per_cu = std::max(1u, std::min((uint32_t)std::max(1, blocks), LDS_PER_CU / LDS_GRANULE / std::max(1u, pieces)));
         resident.store(per_cu, std::memory_order_relaxed);
     }
     const uint32_t waves =
