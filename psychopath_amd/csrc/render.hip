@@ -775,9 +775,9 @@ __global__ __launch_bounds__(KBLOCK) __attribute__((amdgpu_waves_per_eu(MINW))) 
     __shared__ uint32_t app_cnt[2 * (KBLOCK / 64)], app_base[2 * (KBLOCK / 64)];
     const uint32_t n_round = (n + (uint32_t)KBLOCK - 1u) / (uint32_t)KBLOCK * (uint32_t)KBLOCK;
     for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < n_round; i += stride) {
-        // Every field starts defined: with those a path does not use left
-        // undefined, the build for 3 waves per SIMD lost the emission of
-        // light hits.
+        // (Fields a path does not use need no value: with them undefined the
+        // compiler once chose registers for the 3-wave build that it spilled
+        // where lanes were missing, check_spills.py.)
         ShadeOut so{};
         float ptime = 0.0f;
         uint32_t p = 0;
