@@ -375,22 +375,26 @@ int psy_tracer_autotune(psy_tracer* tr, const psy_ray_soa* rays, uint64_t n, psy
     int rc = check_soa(rays, hits);
     if (rc) return rc;
     if (n == 0) return fail(PSY_E_INVALID, "autotune needs rays");
-    std::vector<psy_trace_tuning> cands;
+    // The current shape and the default come first, so the choice is never
+    // one that timed slower than either.  24 waves per CU are more than any
+    // build holds: larger counts would be the same launch timed again.
+    const psy_trace_tuning usual = default_tuning();
+    std::vector<psy_trace_tuning> cands{tr->tuning, usual};
     cands.push_back({PSY_KERNEL_SIMPLE, 1, 1, 8, 4, 0});
-    const uint32_t wpc[] = {8, 12, 16, 24, 32};
+    const uint32_t wpc[] = {8, 12, 16, 24};
     const uint32_t refill[] = {1, 8, 16, 32};
     const uint32_t depth[] = {8, 16, 24};
     for (uint32_t w : wpc)
         for (uint32_t r : refill)
             for (uint32_t dd : depth)
-                for (uint32_t occ : {4u, 8u}) cands.push_back({PSY_KERNEL_PERSISTENT, w, r, dd, occ, 0});
+                for (uint32_t occ : {4u, 8u}) cands.push_back({PSY_KERNEL_PERSISTENT, w, r, dd, occ, usual.leaf_min});
     // The cooperative node fetch (static scenes only; on scenes with time
     // samples it runs as the plain persistent kernel).  Its 7 KB of node
     // staging per wave caps it near 16 resident waves per CU.
     if (!tr->scene->host.has_motion)
         for (uint32_t w : {8u, 12u, 16u})
             for (uint32_t r : {8u, 16u, 32u})
-                for (uint32_t dd : {8u, 16u}) cands.push_back({PSY_KERNEL_PERSISTENT_COOP, w, r, dd, 4u, 0});
+                for (uint32_t dd : {8u, 16u}) cands.push_back({PSY_KERNEL_PERSISTENT_COOP, w, r, dd, 4u, usual.leaf_min});
     const psy_trace_tuning saved = tr->tuning;
     float best_ms = 1e30f;
     psy_trace_tuning best_t = saved;
@@ -418,19 +422,19 @@ int psy_tracer_autotune(psy_tracer* tr, const psy_ray_soa* rays, uint64_t n, psy
         runs += 3 * cands.size();
         return PSY_OK;
     };
-    // Stage 1: kernel, waves, refill, LDS depth and register budget with
-    // per-lane descents; stage 2: the in-loop descents and their threshold
-    // around the best.
+    // Stage 1: kernel, waves, refill, LDS depth and register budget with the
+    // default's descents; stage 2: per-lane descents and the in-loop ones'
+    // threshold around the best.
     rc = time_all();
     if (rc) return rc;
     if (best_t.kernel != PSY_KERNEL_SIMPLE) {
         const psy_trace_tuning s1 = best_t;
         cands.clear();
         const uint32_t k = s1.kernel;
-        for (uint32_t lm : {8u, 16u, 24u, 32u, 48u, 64u})
+        for (uint32_t lm : {0u, 8u, 16u, 24u, 48u, 64u})
             for (uint32_t r : {8u, 16u, 32u})
                 for (uint32_t w : (k == PSY_KERNEL_PERSISTENT_COOP ? std::vector<uint32_t>{8u, 12u, 16u}
-                                                                   : std::vector<uint32_t>{16u, 24u, 32u}))
+                                                                   : std::vector<uint32_t>{16u, 24u}))
                     cands.push_back({k, w, r, s1.stack_lds, s1.simd_waves, lm});
         rc = time_all();
         if (rc) return rc;

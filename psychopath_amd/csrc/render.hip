@@ -1810,14 +1810,29 @@ int psy_renderer_autotune(psy_renderer* r, const psy_camera_desc* cam, const psy
             best_sw = r->shade_waves;
         }
     };
+    // The current choice and the default shape come first, so the result is
+    // never one that timed slower than either.
+    {
+        float ms;
+        rc = time_trial(ms);
+        if (!rc) consider(ms);
+    }
     // Stage 1: the traversal launch shape, sorting on, current shading build.
+    // 24 waves per CU are more than any build holds.
     r->sort_materials = true;
+    const psy_trace_tuning usual = default_tuning();
+    if (!rc) {
+        r->tuning = usual;
+        float ms;
+        rc = time_trial(ms);
+        if (!rc) consider(ms);
+    }
     for (uint32_t sw : {4u, 8u}) {
-        for (uint32_t w : {16u, 24u, 32u}) {
+        for (uint32_t w : {16u, 24u}) {
             for (uint32_t refill : {8u, 16u, 32u}) {
                 for (uint32_t lds : {8u, 16u, 24u}) {
                     if (rc) break;
-                    r->tuning = psy_trace_tuning{PSY_KERNEL_PERSISTENT, w, refill, lds, sw, 0};
+                    r->tuning = psy_trace_tuning{PSY_KERNEL_PERSISTENT, w, refill, lds, sw, usual.leaf_min};
                     float ms;
                     rc = time_trial(ms);
                     if (!rc) consider(ms);
@@ -1826,7 +1841,7 @@ int psy_renderer_autotune(psy_renderer* r, const psy_camera_desc* cam, const psy
         }
     }
     // Stage 1b: the traversal's descent threshold.
-    for (uint32_t lm : {8u, 16u, 32u, 64u}) {
+    for (uint32_t lm : {0u, 8u, 16u, 64u}) {
         if (rc) break;
         r->tuning = best_t;
         r->tuning.leaf_min = lm;

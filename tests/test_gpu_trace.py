@@ -497,6 +497,29 @@ def test_autotune_picks_a_valid_shape(small):
     tr.set_tuning(0, 16, 16, 16, 4, 0)
 
 
+@pytest.mark.parametrize("shape", [(0, 24, 16, 16, 4, 32), (0, 1, 64, 8, 4, 0)])
+def test_autotune_is_not_slower_than_the_shapes_it_starts_from(small, shape):
+    """Neither than the tracer's shape when it is called nor than the default.
+    Kernel times, the least of nine in turn; the margin is the spread of such
+    times (a few per cent) several times over."""
+    v, f, s, o, tr = small
+    r = scenes.incoherent_rays(v.min(0), v.max(0), 200_000, seeds=(151, 152, 153))
+    rays = DeviceRays(ray_batch(r))
+    hits = DeviceHits(rays.n)
+    tr.set_tuning(*shape)
+    best = tuple(tr.autotune(rays, hits).values())
+    assert best[1] <= 24  # (more is the same launch)
+    default = tuple(Tracer(s).tuning().values())
+    ms = {t: [] for t in (best, shape, default)}
+    for _ in range(9):
+        for t in ms:
+            tr.set_tuning(*t)
+            tr.trace_device(rays, hits)
+            ms[t].append(tr.last_kernel_ms())
+    tr.set_tuning(0, 16, 16, 16, 4, 0)
+    assert min(ms[best]) <= 1.2 * min(min(ms[shape]), min(ms[default])), ms
+
+
 def test_time_sampled_light_sizes_match_oracle():
     """Sphere radii and rectangle dimensions as time samples: the trace
     kernels lerp them at each ray's time like the oracle, on rays grazing the
