@@ -259,7 +259,9 @@ typedef struct {
  * leaf or a node whose children all miss, 1..64 pops past such nodes inside
  * the descent and ends a wave's descent round once no lane stands on an
  * internal node or `leaf_min` lanes wait at a leaf.  The simple kernel runs
- * one lane per ray over a launch-wide grid.  No field changes the results. */
+ * one lane per ray over a launch-wide grid.  Scenes of more than 2^25 nodes
+ * run with 16 stack entries in LDS, up to 128 VGPRs and no cooperative fetch
+ * whatever these fields say.  No field changes the results. */
 #define PSY_KERNEL_PERSISTENT 0u
 #define PSY_KERNEL_SIMPLE 1u
 #define PSY_KERNEL_PERSISTENT_COOP 2u
@@ -295,6 +297,10 @@ int psy_scene_create(const psy_scene_desc* desc, psy_scene** out);
 int psy_scene_create_on_device(const psy_scene_desc* desc, uint32_t min_tris, psy_scene** out);
 int psy_scene_destroy(psy_scene* scene);
 int psy_scene_get_info(const psy_scene* scene, psy_scene_info* info);
+/* Test hook: with `on` != 0 the persistent kernels address the scene's nodes
+ * as they do those of a scene with more than 2^25 (4 GB).  Set it before a
+ * renderer is made for the scene.  No result changes. */
+int psy_scene_set_wide_offsets(psy_scene* scene, uint32_t on);
 
 /* Canonical pre-order dump of one host-built BVH4 for parity checks against
  * the reference builder: mesh index, or -1 for the instance BVH.  Writes at

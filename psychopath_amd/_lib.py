@@ -227,6 +227,7 @@ _SIGNATURES = {
     "psy_scene_create": (C.c_int, [C.POINTER(SceneDesc), C.POINTER(C.c_void_p)]),
     "psy_scene_create_on_device": (C.c_int, [C.POINTER(SceneDesc), C.c_uint32, C.POINTER(C.c_void_p)]),
     "psy_scene_destroy": (C.c_int, [C.c_void_p]),
+    "psy_scene_set_wide_offsets": (C.c_int, [C.c_void_p, C.c_uint32]),
     "psy_scene_get_info": (C.c_int, [C.c_void_p, C.POINTER(SceneInfo)]),
     "psy_scene_dump_bvh": (C.c_int64, [C.c_void_p, C.c_int32, _u32p, C.c_uint64, _u32p, C.c_uint64]),
     "psy_tracer_create": (C.c_int, [C.c_void_p, C.c_uint64, C.POINTER(C.c_void_p)]),

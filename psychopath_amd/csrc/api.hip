@@ -68,7 +68,7 @@ TraceArgs scene_args(const psy_scene* s) {
     a.order_table = s->order_table;
     a.groups = s->host.nested ? s->groups : nullptr;
     a.top_root = s->host.top_root;
-    a.node_count = (uint32_t)s->host.nodes.size();
+    a.wide = s->wide_offsets || s->host.nodes.size() > (1u << 25) ? 1u : 0u;  // (a node takes 128 bytes)
     a.odd_boxes = s->host.odd_boxes ? 1u : 0u;
     return a;
 }
@@ -358,6 +358,12 @@ int psy_trace_async(psy_tracer* tr, const psy_ray_soa* rays, uint64_t n, psy_hit
 int psy_tracer_get_tuning(const psy_tracer* tr, psy_trace_tuning* t) {
     if (!tr || !t) return fail(PSY_E_INVALID, "NULL argument");
     *t = tr->tuning;
+    return PSY_OK;
+}
+
+int psy_scene_set_wide_offsets(psy_scene* s, uint32_t on) {
+    if (!s) return fail(PSY_E_INVALID, "scene is NULL");
+    s->wide_offsets = on != 0;
     return PSY_OK;
 }
 

@@ -71,6 +71,7 @@ struct psy_scene {
     psy::GpuGroup* groups = nullptr;
     uint64_t device_bytes = 0;
     bool uploaded = false;
+    bool wide_offsets = false;  // psy_scene_set_wide_offsets
     int device = -1;  // device the scene is resident on
 
     ~psy_scene() {

@@ -37,7 +37,7 @@ struct TraceArgs {
     const uint8_t* order_table;  // visit order of node slots per [octant][code], 8 x 48 bytes
     const GpuGroup* groups;      // nested scenes: instance paths (layout.h), else NULL
     uint32_t top_root;
-    uint32_t node_count;
+    uint32_t wide;               // node addresses need 64-bit offsets
     uint32_t odd_boxes;          // some node's box needs the full test (PackedScene)
     // rays (device)
     const float *ox, *oy, *oz, *dx, *dy, *dz, *time, *max_t;

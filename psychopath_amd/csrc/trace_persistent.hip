@@ -707,7 +707,7 @@ hipError_t launch_one(const TraceArgs& a, unsigned int* work, const TraceTuning&
     // sphere took 1.98 ms so and 1.14 with 100 registers, 1M rays on the
     // motion scene 2.62 and 0.88.
     // The cooperative node fetch serves static single-level scenes.
-    if constexpr (!COUNT && !MOTION && !NESTED) {
+    if constexpr (!COUNT && !MOTION && !NESTED && !BIG) {
         if (tune.coop) {
             if (tune.occupancy >= 8) return launch_resident<&trace_persistent_kernel<false, XF, false, RING, 1, true, false, false, DIRECT>>(a, work, tune, s);
             return launch_resident<&trace_persistent_kernel<false, XF, false, RING, 4, true, false, false, DIRECT>>(a, work, tune, s);
@@ -735,11 +735,17 @@ hipError_t launch_depth(const TraceArgs& a, unsigned int* work, const TraceTunin
 template <bool COUNT>
 hipError_t launch_feat(const TraceArgs& a, unsigned int* work, const TraceTuning& tune, bool xf, bool motion,
                        hipStream_t s) {
-    // More than 4 GB of nodes: the most general build, with 64-bit node
-    // offsets.
-    if (a.node_count > (1u << 25)) {
+    const bool direct = !a.groups && !xf && a.top_root != REF_EMPTY && (a.top_root & REF_LEAF);
+    // More than 4 GB of nodes: builds with 64-bit node offsets, by the same
+    // features (in one build for all of them, 4.2M rays on the 1M-triangle
+    // sphere addressed so took 1.63 ms and 1.08 in the static one, 1M rays on
+    // the large instanced scene 0.59 and 0.50).
+    if (a.wide) {
         if (a.groups) return launch_one<COUNT, true, true, 16, true, true, false>(a, work, tune, s);
-        return launch_one<COUNT, true, true, 16, false, true, false>(a, work, tune, s);
+        if (motion) return launch_one<COUNT, true, true, 16, false, true, false>(a, work, tune, s);
+        if (xf) return launch_one<COUNT, true, false, 16, false, true, false>(a, work, tune, s);
+        if (direct) return launch_one<COUNT, false, false, 16, false, true, true>(a, work, tune, s);
+        return launch_one<COUNT, false, false, 16, false, true, false>(a, work, tune, s);
     }
     // Nested scenes take the transform path, with or without time samples.
     if (a.groups) {
@@ -748,7 +754,6 @@ hipError_t launch_feat(const TraceArgs& a, unsigned int* work, const TraceTuning
     }
     if (xf && motion) return launch_depth<COUNT, true, true, false, false>(a, work, tune, s);
     if (xf) return launch_depth<COUNT, true, false, false, false>(a, work, tune, s);
-    const bool direct = a.top_root != REF_EMPTY && (a.top_root & REF_LEAF);
     if (motion && direct) return launch_depth<COUNT, false, true, false, true>(a, work, tune, s);
     if (motion) return launch_depth<COUNT, false, true, false, false>(a, work, tune, s);
     if (direct) return launch_depth<COUNT, false, false, false, true>(a, work, tune, s);

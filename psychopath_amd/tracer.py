@@ -237,6 +237,11 @@ class Scene:
         check("psy_scene_get_info", lib().psy_scene_get_info(self.handle, C.byref(i)))
         return {f: getattr(i, f) for f, _ in _lib.SceneInfo._fields_}
 
+    def wide_offsets(self, on: bool = True) -> None:
+        """Test hook (psy_scene_set_wide_offsets): traverse as scenes above
+        2^25 nodes are."""
+        check("psy_scene_set_wide_offsets", lib().psy_scene_set_wide_offsets(self.handle, int(on)))
+
     def dump_bvh(self, mesh: int) -> tuple[np.ndarray, np.ndarray]:
         """Canonical dump of a mesh BVH4 (mesh >= 0) or the instance BVH
         (mesh = -1), and the object order of its leaves."""
