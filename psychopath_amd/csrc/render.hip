@@ -1571,9 +1571,13 @@ int psy_renderer_create(const psy_scene* scene_c, const psy_world_desc* world, u
     // The colours that shading evaluates again and again, laid out once:
     // the shaders', the background, and lights' without time samples.
     {
-        std::vector<GpuColor> colors;
-        for (const GpuClosure& c : shaders) colors.push_back(c.color);
-        colors.push_back(sc.background);
+        std::vector<GpuColor> colors{sc.background};
+        std::vector<uint32_t> prepared;  // the shaders whose colours follow
+        for (uint32_t i = 0; i < shaders.size() && prepared.size() < PREPARED_SHADERS; i++)
+            if (shaders[i].color.kind == PSY_COLOR_XYZ) {
+                prepared.push_back(i);
+                colors.push_back(shaders[i].color);
+            }
         const uint32_t fixed = (uint32_t)colors.size();
         const std::vector<GpuRectLight>& rl = scene->host.rect_lights;
         const std::vector<GpuSphereLight>& sl = scene->host.sphere_lights;
@@ -1595,9 +1599,8 @@ int psy_renderer_create(const psy_scene* scene_c, const psy_world_desc* world, u
         if (e != hipSuccess) return bail(fail(PSY_E_DEVICE, std::string("colour set-up: ") + hipGetErrorString(e)));
         r->release(dcol);
         sc.light_colors = prep + fixed;
-        for (size_t i = 0; i < shaders.size(); i++)
-            if (shaders[i].color.kind == PSY_COLOR_XYZ) shaders[i].color = prepared_ref(prep + i);
-        if (sc.background.kind == PSY_COLOR_XYZ) sc.background = prepared_ref(prep + shaders.size());
+        for (size_t k = 0; k < prepared.size(); k++) shaders[prepared[k]].color = prepared_ref(prep + 1 + k);
+        if (sc.background.kind == PSY_COLOR_XYZ) sc.background = prepared_ref(prep);
     }
     rc = r->alloc(&dsh, shaders.size());
     if (!rc) rc = r->alloc(&ddl, distant.size());

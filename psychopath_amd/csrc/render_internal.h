@@ -22,9 +22,9 @@ using rd::HaltonDim;
 
 constexpr int KBLOCK = 256;
 constexpr uint32_t MAX_SEGS = 64;  // requests interleaved in one wave
-// Lights whose colours a renderer prepares, 1.5 KB each; the others' are
-// evaluated from the shared tables.
-constexpr uint32_t PREPARED_LIGHTS = 4096;
+// Lights and shaders whose colours a renderer prepares, 1.5 KB each; the
+// others' are evaluated from the shared tables.
+constexpr uint32_t PREPARED_LIGHTS = 4096, PREPARED_SHADERS = 4096;
 constexpr uint32_t NUM_BINS = 6;   // miss, light, Lambert, GGX, emit, dielectric
 // Layout of the renderer's counter words: [0, 4) queue counts, then the sort
 // bins (NUM_BINS), then the rays-traced u64 at an even word.
