@@ -1010,18 +1010,12 @@ void halton_tables(std::vector<HaltonDim>& dims, std::vector<uint16_t>& perms) {
     perms.clear();
     for (int i = 1; i < NUM; i++) {
         const uint64_t base = primes[i];
-        uint64_t digits = 1, pow_base = base;
-        while (pow_base * base <= 500) {
-            pow_base *= base;
-            digits++;
-        }
-        uint64_t max_power = pow_base;
-        while (max_power * pow_base < (1ull << 32)) max_power *= pow_base;
-        HaltonDim d{(uint32_t)base, (uint32_t)pow_base, (uint32_t)max_power, (uint32_t)perms.size()};
-        for (uint64_t j = 0; j < pow_base; j++) {
+        const HaltonPowers p = halton_powers(primes[i]);
+        HaltonDim d{primes[i], p.pow_base, p.max_power, (uint32_t)perms.size()};
+        for (uint64_t j = 0; j < p.pow_base; j++) {
             // Digits of j, least significant first, permuted and reversed.
             uint64_t idx = j, r = 0;
-            for (uint64_t k = 0; k < digits; k++) {
+            for (uint64_t k = 0; k < p.digits; k++) {
                 r = r * base + faure[base][idx % base];
                 idx /= base;
             }

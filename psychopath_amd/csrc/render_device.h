@@ -150,21 +150,28 @@ RD float hash_u32_to_f32(uint32_t n, uint32_t seed) {
 struct HaltonDim {
     uint32_t base, pow_base, max_power, perm_off;
 };
-// pow_base and max_power of the dimensions the renderer samples (base 3, 5,
-// ... 19), as halton_tables computes them: where the dimension is known when
-// compiling, so are the divisors, and a digit group costs a multiplication
-// instead of two integer divisions.  With that and the early end below the
+// The digit groups of a base: base^digits = pow_base <= 500, and the largest
+// power of pow_base below 2^32.
+struct HaltonPowers {
+    uint32_t digits, pow_base, max_power;
+};
+constexpr HaltonPowers halton_powers(uint32_t base) {
+    uint64_t digits = 1, pow_base = base;
+    while (pow_base * base <= 500) {
+        pow_base *= base;
+        digits++;
+    }
+    uint64_t max_power = pow_base;
+    while (max_power * pow_base < (1ull << 32)) max_power *= pow_base;
+    return HaltonPowers{(uint32_t)digits, (uint32_t)pow_base, (uint32_t)max_power};
+}
+// Those of the dimensions the renderer samples: where the dimension is known
+// when compiling, so are the divisors, and a digit group costs a
+// multiplication instead of two integer divisions.  With that and the early end below the
 // Cornell box at 512x512, 16 spp takes 7.05 ms instead of 7.50 and the large
 // scene at full HD, 2 spp, 9.9 instead of 10.05.
-constexpr uint32_t HALTON_POW_BASE[8] = {0, 243, 125, 343, 121, 169, 289, 361};
-constexpr uint32_t HALTON_MAX_POWER[8] = {0,
-                                          243u * 243u * 243u * 243u,
-                                          125u * 125u * 125u * 125u,
-                                          343u * 343u * 343u,
-                                          121u * 121u * 121u * 121u,
-                                          169u * 169u * 169u * 169u,
-                                          289u * 289u * 289u,
-                                          361u * 361u * 361u};
+constexpr HaltonPowers HALTON_FIRST[8] = {{0, 0, 0},         halton_powers(3),  halton_powers(5),  halton_powers(7),
+                                          halton_powers(11), halton_powers(13), halton_powers(17), halton_powers(19)};
 RD float halton_sample(const HaltonDim* dims, const uint16_t* perms, uint32_t dimension, uint32_t index) {
     if (dimension == 0) {
         // Base 2: the bit-reversed index (build.rs:110-126).
@@ -179,8 +186,8 @@ RD float halton_sample(const HaltonDim* dims, const uint16_t* perms, uint32_t di
         return (float)__builtin_bitreverse32(index) * (1.0f / 4294967296.0f);
 #endif
     }
-    const uint32_t pow_base = dimension < 8 ? HALTON_POW_BASE[dimension] : dims[dimension].pow_base;
-    const uint32_t max_power = dimension < 8 ? HALTON_MAX_POWER[dimension] : dims[dimension].max_power;
+    const uint32_t pow_base = dimension < 8 ? HALTON_FIRST[dimension].pow_base : dims[dimension].pow_base;
+    const uint32_t max_power = dimension < 8 ? HALTON_FIRST[dimension].max_power : dims[dimension].max_power;
     const uint16_t* perm = perms + dims[dimension].perm_off;
     // The permutations keep digit zero (Faure's do), so groups above the
     // index's last add nothing: a sample below pow_base takes one look-up.
