@@ -153,7 +153,7 @@ void trace_persistent_kernel(TraceArgs a, unsigned int* work, uint32_t refill_mi
     }
     // A scene that is one untransformed instance needs no walk to it: its rays
     // start on the mesh's root.  That saves every ray a leaf round with two
-    // dependent loads and is worth the four registers (100 instead of 96, so
+    // dependent loads and is worth the two registers (98 instead of 96, so
     // 16 waves per CU instead of 20): 16.7M incoherent rays on the
     // 1M-triangle sphere 3.39 -> 3.24 ms, 4.0M shadow rays 0.943 -> 0.895.  A
     // build of its own, so that other static scenes keep their waves: 4.2M
@@ -510,7 +510,7 @@ void trace_persistent_kernel(TraceArgs a, unsigned int* work, uint32_t refill_mi
                     }
                 }
                 cur = REF_EMPTY;
-            } else if (!in_inst) {
+            } else if (!DIRECT && !in_inst) {
                 // Instance leaf (tracer.rs:95-128).
                 const GpuInstance inst = a.instances[ii];
                 const GpuMesh mesh = a.meshes[inst.mesh];
@@ -700,11 +700,11 @@ hipError_t launch_resident(const TraceArgs& a, unsigned int* work, const TraceTu
 template <bool COUNT, bool XF, bool MOTION, uint32_t RING, bool NESTED, bool BIG, bool DIRECT>
 hipError_t launch_one(const TraceArgs& a, unsigned int* work, const TraceTuning& tune, hipStream_t s) {
     // Register budget: at most 128 VGPRs (four waves per SIMD), or what the
-    // compiler takes of its own (96 to 100 in static builds, 126 with
+    // compiler takes of its own (96 and 98 in static builds, 126 with
     // transforms, up to 152 with time samples as well, which leaves three
     // waves).  A budget of eight waves, 64 VGPRs, would spill in the node
     // step: at 24 waves per CU and leaf_min 32, 4.2M rays on the 1M-triangle
-    // sphere took 1.98 ms so and 1.14 with 100 registers, 1M rays on the
+    // sphere took 1.98 ms so and 1.13 with 98 registers, 1M rays on the
     // motion scene 2.62 and 0.88.
     // The cooperative node fetch serves static single-level scenes.
     if constexpr (!COUNT && !MOTION && !NESTED && !BIG) {
