@@ -12,12 +12,13 @@ form of the reference's returned SurfaceIntersection slice.  The launch shape
 is autotuned on a second ray set from the same generator with other seeds,
 then the benchmark rays are timed.
 
-Prints one JSON line.  `roofline` models the traversal kernel's algorithmic
-bytes: per ray, internal-node visits x 112 B (the seven 16-B parts of a
-128-B node record that a node without time samples needs: child boxes and
-references) + triangle tests x 48 B triangle record + 65 B of ray and hit
-I/O (33 B ray in, 32 B record out), with visit counts from an instrumented
-run of the same kernel on the same rays.  `cpu_baseline` times the oracle (a C++ restatement of the
+Prints one JSON line.  `roofline` models what bounds the traversal kernel, L1
+tag lookups: per ray, internal-node visits x 7 (the 16-B parts of a 128-B node
+record that a node without time samples needs: child boxes and references) +
+triangle tests x 3 (a 48-B record), one lookup each, with visit counts from an
+instrumented run of the same kernel on the same rays.  The bytes that pass
+through the L1 so (with 65 B of ray and hit I/O: 33 B ray in, 32 B record out)
+mostly come from the caches; `traffic` is what reached HBM.  `cpu_baseline` times the oracle (a C++ restatement of the
 reference's ray-stream tracer, batches of 4096 rays, one tracer per thread)
 on a sample of the same rays, on the host cores allotted to this process.
 """
@@ -33,6 +34,7 @@ sys.path.insert(0, ROOT)
 
 METRIC = "incoherent Mrays/s on 1M-tri BVH4; samples/s + p50/p99 latency served vs plain"
 HBM_PEAK_GBS = 8000.0
+L1_PEAK_GLOOKUPS = 614.4     # 256 CUs, one tag lookup a clock each, 2.4 GHz
 RAY_IN_BYTES = 8 * 4 + 1     # ox oy oz dx dy dz time max_t + flags
 HIT_OUT_BYTES = 32           # one psy_hit_record: t b0 b1 b2 prim inst kind reserved
 STATIC_NODE_READ_BYTES = 112  # 96 B child boxes + 16 B child references of a 128-B node
@@ -210,7 +212,9 @@ def main():
     avg_kernel_ms = float(np.mean(kernel_ms))
     log(f"timed {args.steps} steps: {ms_per_step:.2f} ms/step, kernel {avg_kernel_ms:.2f} ms, {mrays:.1f} Mrays/s")
 
-    # Algorithmic bytes per launch from the instrumented kernel.
+    # Visits per launch from the instrumented kernel.  A lane's 16-byte part
+    # of a node or triangle is one L1 tag lookup, of which a CU makes one a
+    # clock; most of the bytes come from the caches, so HBM is no bound.
     counts = tracer.trace_counted(d_rays, d_hits)
     h = d_hits.to_host()
     hit_frac = float((h.kind == 2).mean())
@@ -219,6 +223,7 @@ def main():
     io_b = RAY_IN_BYTES + HIT_OUT_BYTES
     alg_bytes = counts["node_visits"] * node_b + counts["tri_tests"] * tri_b + args.rays * io_b
     achieved = alg_bytes / (avg_kernel_ms * 1e-3) / 1e9
+    lookups = counts["node_visits"] * (node_b // 16) + counts["tri_tests"] * (tri_b // 16)
 
     # HBM traffic per launch, from the committed rocprofv3 --pmc summary of
     # this benchmark's kernel (L2-to-memory requests by size, cross-checked
@@ -312,13 +317,18 @@ def main():
             "bvh_depth": info["max_depth"],
         },
         "roofline": {
-            "bound": "hbm",
-            "achieved": round(achieved, 1),
-            "peak": HBM_PEAK_GBS,
-            "unit": "GB/s",
-            "frac": round(achieved / HBM_PEAK_GBS, 4),
+            "bound": "l1",
+            "achieved": round(lookups / (avg_kernel_ms * 1e-3) / 1e9, 1),
+            "peak": L1_PEAK_GLOOKUPS,
+            "unit": "Glookups/s",
+            "frac": round(lookups / (avg_kernel_ms * 1e-3) / 1e9 / L1_PEAK_GLOOKUPS, 4),
+            "lookups_model": f"node_visits*{node_b // 16} + tri_tests*{tri_b // 16}",
+            "bytes_through_l1_gb_per_s": round(achieved, 1),
             "traffic": traffic,
             "traffic_source": traffic_info,
+            "traffic_gb_per_s": None if traffic is None else round(
+                traffic / (traffic_info["profiled_kernel_ms"] * 1e-3) / 1e9, 1),
+            "hbm_peak_gb_per_s": HBM_PEAK_GBS,
             "kernel": {0: "trace_persistent_kernel", 1: "trace_kernel",
                        2: "trace_persistent_kernel (cooperative node fetch)"}[tuning["kernel"]],
             "kernel_ms": round(avg_kernel_ms, 3),
@@ -349,7 +359,7 @@ RENDER_BYTES = {
     "shadow_ray": 33,     # per shadow ray: ray in + hit kind out
     "instance": 80,       # per instance entry: instance record + one transform
     "shadow": 49,         # per shadow result, added by the shading step: kind, pending and colour in, colour out
-    "sort": 14,           # per closest hit: kind and instance twice, order out
+    "sort": 9,            # per closest hit: kind and instance, order out
     "shade": 310,         # per closest hit: path state in/out, hit, ray, triangle and instance records, 2 queued rays
     "film": 68,           # per path: colour and wavelength in, XYZ out and in, film read-modify-write
 }
@@ -379,7 +389,9 @@ def render_roofline(prof: dict, cnt: dict, node_b: int, tri_b: int) -> dict:
         out[k] = {"ms": round(ms, 3), "bytes": int(by), "achieved": round(gbs, 1),
                   "frac": round(gbs / HBM_PEAK_GBS, 4)}
     ach = tot_b / (tot_ms * 1e-3) / 1e9 if tot_ms > 0 else 0.0
-    return {"bound": "hbm", "achieved": round(ach, 1), "peak": HBM_PEAK_GBS, "unit": "GB/s",
+    # (the stages wait for their longest rays and for gathers; the share of the
+    # HBM peak says how far below it they run)
+    return {"bound": "latency", "achieved": round(ach, 1), "peak": HBM_PEAK_GBS, "unit": "GB/s",
             "frac": round(ach / HBM_PEAK_GBS, 4), "traffic": None, "device_ms": round(tot_ms, 3),
             "algorithmic_bytes": int(tot_b), "stages": out,
             "counts": {k: int(prof[k]) for k in ("paths", "closest_rays", "shadow_rays")} |
