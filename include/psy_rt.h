@@ -250,15 +250,17 @@ typedef struct {
  * scenes without time samples (elsewhere it runs as the persistent kernel).
  * The persistent kernel keeps
  * `waves_per_cu` wave64 workgroups per compute unit resident (at most as
- * many as its registers and LDS let a unit hold), each starting
- * on its share of the rays and then taking chunks from a counter; lanes whose ray finished are
- * refilled from the wave's chunk once `refill_min` lanes of a wave are idle; `stack_lds` stack entries per lane
- * live in LDS (8, 16, or 24 for a ring of 32) and the rest in private memory;
- * `simd_waves` is the register budget (4: up to 128 VGPRs, for four waves per
- * SIMD at least; 8: the compiler's choice, for three to five); `leaf_min` 0 lets each lane descend until it reaches a
- * leaf or a node whose children all miss, 1..64 pops past such nodes inside
- * the descent and ends a wave's descent round once no lane stands on an
- * internal node or `leaf_min` lanes wait at a leaf.  The simple kernel runs
+ * many as its registers and LDS let a unit hold, 9 to 20; the field keeps what
+ * was asked for), each starting on its share of the rays and then taking
+ * chunks from a counter; lanes whose ray finished are refilled from the wave's
+ * chunk once `refill_min` lanes of a wave are idle; `stack_lds` stack entries
+ * per lane live in LDS (8, 16, or 24 for a ring of 32) and the rest in private
+ * memory; `simd_waves` is the register budget (4: up to 128 VGPRs, for four
+ * waves per SIMD at least; 8: the compiler's choice, for three to five);
+ * `leaf_min` 0 lets each lane descend until it reaches a leaf or a node whose
+ * children all miss, 1..64 pops past such nodes inside the descent and ends a
+ * wave's descent round once no lane stands on an internal node or `leaf_min`
+ * lanes wait at a leaf.  The simple kernel runs
  * one lane per ray over a launch-wide grid.  Scenes of more than 2^25 nodes
  * run with 16 stack entries in LDS, up to 128 VGPRs and no cooperative fetch
  * whatever these fields say.  No field changes the results. */
